@@ -42,7 +42,7 @@
 //     same carry, but selects the writing block by `(block+1) * RADIX_DIGITS >= n`,
 //     agent/agent_radix_sort_onesweep.h:362, so it never fires for large inputs.)
 // Algorithmic traffic per pass: n * 2 * (sizeof(K) + sizeof(V)) bytes; the histogram reads n*sizeof(K).
-#include "common.hpp"
+#include "radix_keys.hpp"
 #include "../../include/lcpp_hip.h"
 
 #include <algorithm>
@@ -70,51 +70,6 @@ constexpr uint32_t ballot_sixteenths_for(int mode, uint32_t mixed) {
 __device__ uint64_t* g_trace_buffer = nullptr;
 __device__ uint64_t g_trace_records = 0;
 #endif
-
-enum KeyKind { kUnsigned = 0, kSigned = 1, kFloat = 2 };
-
-template <typename K> struct KeyTraits;
-template <> struct KeyTraits<uint32_t> { using U = uint32_t; static constexpr int kind = kUnsigned; };
-template <> struct KeyTraits<int32_t> { using U = uint32_t; static constexpr int kind = kSigned; };
-template <> struct KeyTraits<float> { using U = uint32_t; static constexpr int kind = kFloat; };
-template <> struct KeyTraits<uint64_t> { using U = uint64_t; static constexpr int kind = kUnsigned; };
-template <> struct KeyTraits<int64_t> { using U = uint64_t; static constexpr int kind = kSigned; };
-template <> struct KeyTraits<double> { using U = uint64_t; static constexpr int kind = kFloat; };
-
-template <int VB> struct ValueWord { using type = uint32_t; };
-template <> struct ValueWord<8> { using type = uint64_t; };
-
-// Bit-ordered transform (common/util_type.h:97-175 TwiddleIn/TwiddleOut; descending inverts,
-// agent/radix_rank_sort_operations.h:123-155).
-template <typename U, int KIND, bool DESC>
-__device__ __forceinline__ U twiddle_in(U k) {
-    constexpr U kHigh = U(1) << (sizeof(U) * 8 - 1);
-    if constexpr (KIND == kSigned) k ^= kHigh;
-    if constexpr (KIND == kFloat) k ^= (k & kHigh) ? U(~U(0)) : kHigh;
-    if constexpr (DESC) k = ~k;
-    return k;
-}
-
-template <typename U, int KIND, bool DESC>
-__device__ __forceinline__ U twiddle_out(U k) {
-    constexpr U kHigh = U(1) << (sizeof(U) * 8 - 1);
-    if constexpr (DESC) k = ~k;
-    if constexpr (KIND == kSigned) k ^= kHigh;
-    if constexpr (KIND == kFloat) k ^= (k & kHigh) ? kHigh : U(~U(0));
-    return k;
-}
-
-// Digit of a bit-ordered key.  For floats the ordered image of -0.0 is mapped to that of +0.0
-// before extraction (ShiftDigitExtractor / ProcessFloatMinusZero,
-// agent/radix_rank_sort_operations.h:31-62), so both zeros rank as equal keys.
-template <typename U, int KIND>
-__device__ __forceinline__ uint32_t digit_of(U ordered, uint32_t shift, uint32_t mask) {
-    if constexpr (KIND == kFloat) {
-        constexpr U kHigh = U(1) << (sizeof(U) * 8 - 1);
-        if (ordered == U(~kHigh)) ordered = kHigh;
-    }
-    return static_cast<uint32_t>(ordered >> shift) & mask;
-}
 
 // The same digit from the bit count of the pass: one bit-field extract for 4-byte keys.
 template <typename U, int KIND>
@@ -1327,6 +1282,21 @@ int sort_entry(void* temp, size_t temp_bytes, const K* keys_in, K* keys_out, con
     void* db_values[2] = {vdb0, vdb1};
     const int sel = db ? *selector : 0;
     int st;
+    // Small inputs: a handful of workgroups sort in LDS (radix_small.hip).  The test hooks that shape the
+    // onesweep passes keep a call on them.  A DoubleBuffer result lands where the passes would leave it: in
+    // the current buffer after an even number of them, else in the other one, and the runs go to the buffer
+    // that the result does not (in place when that is the current one: a tile is read before it is written).
+    // A copy-form sort of one pass has no scratch keys, so above one tile it stays with its one pass.
+    if (portion_limit == 0 && L.rank_mode == kRankMixed && !g_precount.load(std::memory_order_relaxed) &&
+        n <= small_sort_max(sizeof(K)) && (n <= kSmallOneTile || db || keys_tmp)) {
+        const int to = sel ^ static_cast<int>(L.passes & 1u);
+        st = db ? small_sort<K, VB>(db_keys[sel], db_keys[to], db_values[sel], db_values[to], db_keys[to ^ 1],
+                                    db_values[to ^ 1], n, begin_bit, end_bit, descending != 0, stream)
+                : small_sort<K, VB>(keys_in, keys_out, values_in, values_out, keys_tmp, values_tmp, n, begin_bit,
+                                    end_bit, descending != 0, stream);
+        if (st == kOk && db) *selector = to;
+        return st;
+    }
     if (descending)
         st = launch_sort<K, true, VB>(t, L, keys_in, keys_out, values_in, values_out, keys_tmp, values_tmp,
                                       db ? db_keys : nullptr, db ? db_values : nullptr, sel, n, begin_bit, end_bit, stream);
