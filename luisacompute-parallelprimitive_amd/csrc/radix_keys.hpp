@@ -74,5 +74,27 @@ template <typename K, int VB>
 int small_sort(const K* keys_in, K* keys_out, const void* values_in, void* values_out, K* runs_keys, void* runs_values,
                uint32_t n, uint32_t begin_bit, uint32_t end_bit, bool descending, hipStream_t stream);
 
+// mid_sort (radix_mid.hip): onesweep passes with every tile resident, for up to kMidSortMax items.
+constexpr uint32_t kMidSortMax = 1u << 21;
+constexpr int kMidItems = 4;
+constexpr uint32_t kMidTile = 1024 * kMidItems;
+// Tiles per group of the two-level sums: one level up to 32 tiles (100,003 keys 35.1 us per call, 37.9 with groups
+// of 16), then groups of 16 (262,144 keys 40.9 us, 46.1 with groups of 32).
+constexpr uint32_t mid_group(uint32_t tiles) { return tiles <= 32 ? 32u : 16u; }
+struct MidPlan {
+    uint32_t passes;
+    uint32_t tiles;    // of kMidTile keys
+    uint32_t group;    // tiles per group
+    uint32_t rows;     // histogram workgroups, per_row keys each
+    uint32_t per_row;
+    uint32_t* bins;       // passes x 256
+    uint32_t* lookback;   // tiles x 256
+    uint32_t* row_words;  // rows x passes x 256, in memory that pass 0 does not write
+};
+template <typename K, int VB>
+int mid_sort(const MidPlan& plan, const K* keys_in, K* keys_out, const void* values_in, void* values_out, K* keys_tmp,
+             void* values_tmp, uint32_t n, uint32_t begin_bit, uint32_t end_bit, bool descending, uint32_t spin_limit,
+             hipStream_t stream);
+
 }  // namespace radix
 }  // namespace lcpp_hip

@@ -3,7 +3,8 @@
 //
 // The onesweep path of a few thousand keys spends its time on launches and on one tile's chain of dependent
 // LDS round trips per pass (seven launches, 16-19 us per pass at 20,011 pairs), with all but one or two CUs
-// idle: 20,011 f32 + u32 pairs took 83 us per call, 2,000 u32 pairs 68; 16.5 and 8.4.  Every pass of a tile runs in LDS inside one launch:
+// idle: 83 us per call of 20,011 f32 + u32 pairs, 68 of 2,000 u32 + u32 pairs; here 16.5 and 8.4.  Every pass
+// of a tile runs in LDS inside one launch:
 //   * up to kSmallOneTile items: one workgroup sorts them all and writes the output.
 //   * up to small_sort_max items: tiles of kRunItems items are sorted by one workgroup each into the scratch
 //     buffer; then every item's output position is its index in its run plus, for every other run, the

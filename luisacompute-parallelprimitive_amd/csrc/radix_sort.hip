@@ -1104,6 +1104,12 @@ HistPlan hist_plan(uint32_t len, uint32_t granule = hist_step<K>(), bool tiles =
     return HistPlan{per, static_cast<unsigned>(ceil_div(len, per))};
 }
 
+// Medium sorts (radix_mid.hip).
+// At most kMidRows histogram workgroups (every tile of pass 0 adds up their rows; 128 of 4,096 keys: 63.0 us per
+// call of 1,000,003 pairs against 59.8), each with at least kMidRowItems keys.
+constexpr uint32_t kMidRows = 64;
+constexpr uint32_t kMidRowItems = 8192;
+
 template <typename K, bool DESC, int VB>
 int launch_sort(char* temp, const Layout& L, const K* keys_in, K* keys_out, const void* values_in, void* values_out,
                 K* keys_tmp, void* values_tmp, K* const* db_keys, void* const* db_values, int sel, uint32_t n,
@@ -1225,6 +1231,52 @@ int launch_sort(char* temp, const Layout& L, const K* keys_in, K* keys_out, cons
     return kOk;
 }
 
+// The plan of a medium sort and its place in the temp storage: bins, look-back rows, scratch keys and values
+// (`tmp_at`, copy form), then the histogram rows; where only the latter do not fit, a copy-form sort keeps them
+// in the one of its two destinations that pass 0 does not write (the histogram and pass 0 also read the
+// inputs, so not in an output that overlaps them).  False if there is no room.
+template <typename K, int VB>
+bool mid_plan(uint32_t n, uint32_t passes, bool db, char* temp, size_t temp_bytes, const K* keys_in, K* keys_out,
+              const void* values_in, MidPlan& M, char*& tmp_at) {
+    M.passes = passes;
+    M.tiles = static_cast<uint32_t>(ceil_div(n, kMidTile));
+    M.group = mid_group(M.tiles);
+    M.rows = static_cast<uint32_t>(std::min<uint64_t>(kMidRows, ceil_div(n, kMidRowItems)));
+    M.per_row = static_cast<uint32_t>(ceil_div(n, M.rows));
+    size_t off = align_up(static_cast<size_t>(passes) * kDigits * 4, kViewAlign);
+    const size_t lookback_off = off;
+    off += static_cast<size_t>(M.tiles) * kDigits * 4;
+    const size_t tmp_off = off;
+    const size_t key_bytes = static_cast<size_t>(n) * sizeof(K);
+    if (!db && passes > 1) {
+        off += key_bytes;
+        if (VB) off = align_up(off, kViewAlign) + static_cast<size_t>(n) * VB;
+    }
+    if (temp_bytes < off) return false;
+    const size_t row_bytes = static_cast<size_t>(M.rows) * passes * kDigits * 4;
+    M.bins = reinterpret_cast<uint32_t*>(temp);
+    M.lookback = reinterpret_cast<uint32_t*>(temp + lookback_off);
+    tmp_at = temp + tmp_off;
+    off = align_up(off, kViewAlign);
+    if (temp_bytes >= off + row_bytes) {
+        M.row_words = reinterpret_cast<uint32_t*>(temp + off);
+        return true;
+    }
+    if (db || passes == 1 || row_bytes > key_bytes) return false;
+    if (passes % 2 == 1) {  // pass 0 writes the output
+        M.row_words = reinterpret_cast<uint32_t*>(tmp_at);
+        return true;
+    }
+    const char* out = reinterpret_cast<const char*>(keys_out);
+    auto apart = [&](const void* in, size_t bytes) {
+        const char* i = static_cast<const char*>(in);
+        return i + bytes <= out || out + key_bytes <= i;
+    };
+    if (!apart(keys_in, key_bytes) || (VB && !apart(values_in, static_cast<size_t>(n) * VB))) return false;
+    M.row_words = reinterpret_cast<uint32_t*>(keys_out);
+    return true;
+}
+
 template <typename K, int VB>
 int sort_entry(void* temp, size_t temp_bytes, const K* keys_in, K* keys_out, const void* values_in, void* values_out,
                K* db0, K* db1, void* vdb0, void* vdb1, int* selector, uint32_t n, uint32_t begin_bit, uint32_t end_bit,
@@ -1287,15 +1339,31 @@ int sort_entry(void* temp, size_t temp_bytes, const K* keys_in, K* keys_out, con
     // the current buffer after an even number of them, else in the other one, and the runs go to the buffer
     // that the result does not (in place when that is the current one: a tile is read before it is written).
     // A copy-form sort of one pass has no scratch keys, so above one tile it stays with its one pass.
-    if (portion_limit == 0 && L.rank_mode == kRankMixed && !g_precount.load(std::memory_order_relaxed) &&
-        n <= small_sort_max(sizeof(K)) && (n <= kSmallOneTile || db || keys_tmp)) {
-        const int to = sel ^ static_cast<int>(L.passes & 1u);
+    const bool hooked = portion_limit != 0 || L.rank_mode != kRankMixed || g_precount.load(std::memory_order_relaxed);
+    const int to = sel ^ static_cast<int>(L.passes & 1u);
+    if (!hooked && n <= small_sort_max(sizeof(K)) && (n <= kSmallOneTile || db || keys_tmp)) {
         st = db ? small_sort<K, VB>(db_keys[sel], db_keys[to], db_values[sel], db_values[to], db_keys[to ^ 1],
                                     db_values[to ^ 1], n, begin_bit, end_bit, descending != 0, stream)
                 : small_sort<K, VB>(keys_in, keys_out, values_in, values_out, keys_tmp, values_tmp, n, begin_bit,
                                     end_bit, descending != 0, stream);
         if (st == kOk && db) *selector = to;
         return st;
+    }
+    // Medium inputs: passes whose tiles are all resident (radix_mid.hip), when the temp storage has room for
+    // their look-back rows (a reference-sized one does).
+    if (!hooked && n <= kMidSortMax) {
+        MidPlan M;
+        char* tmp_at = nullptr;
+        if (mid_plan<K, VB>(n, L.passes, db, t, temp_bytes, keys_in, keys_out, values_in, M, tmp_at)) {
+            K* mid_keys_tmp = reinterpret_cast<K*>(tmp_at);
+            void* mid_values_tmp = VB ? tmp_at + align_up(static_cast<size_t>(n) * sizeof(K), kViewAlign) : nullptr;
+            st = db ? mid_sort<K, VB>(M, db_keys[sel], db_keys[to], db_values[sel], db_values[to], db_keys[to ^ 1],
+                                      db_values[to ^ 1], n, begin_bit, end_bit, descending != 0, L.spin_limit, stream)
+                    : mid_sort<K, VB>(M, keys_in, keys_out, values_in, values_out, mid_keys_tmp, mid_values_tmp, n,
+                                      begin_bit, end_bit, descending != 0, L.spin_limit, stream);
+            if (st == kOk && db) *selector = to;
+            return st;
+        }
     }
     if (descending)
         st = launch_sort<K, true, VB>(t, L, keys_in, keys_out, values_in, values_out, keys_tmp, values_tmp,
