@@ -11,7 +11,7 @@
 // leaves a DoubleBuffer untouched.  Any stable sort by the same order gives the same output, so the
 // sort here is free to differ from the reference's merge passes.
 //
-// MI355X design:
+// MI355X design (radix orders with many short segments, and value orders; see wave_route for the others):
 //   * Block phase: chunks sorted in LDS by one 256-thread workgroup each, C = 4,096 items in radix
 //     order and 2,048 in value order.  Tiny segments (<= 16 items) are sorted by one thread each, in
 //     registers; small ones (<= 512 items) together per 2,048-item tile of the item range (a joint sort
@@ -34,7 +34,7 @@
 //     value order (floats of DeviceSegmentedSort) compares the values, so -0.0 equals +0.0.
 // Algorithmic traffic: 2 * (sizeof(K) + sizeof(V)) per item in segments up to C items, plus the
 // same per global pass for longer segments.
-#include "common.hpp"
+#include "segsort_waves.hpp"
 #include "../../include/lcpp_hip.h"
 
 #include <map>
@@ -906,6 +906,15 @@ uint32_t* longest_word(hipStream_t stream) {
     return w;
 }
 
+// Radix order with at least kWaveMean items per segment on average: a wave or a workgroup per segment
+// (segsort_waves.hip), which is faster from there on (per call, here and there: 4 M u32 + u32 pairs of mean 300
+// 203.8 -> 139.6 us, of mean 100 179.9 -> 129.7; 2^26 u32 of mean 100 1,136 -> 922, but of mean 40 953 -> 1,060,
+// where the joint sort of a tile fills its lanes better).
+constexpr uint64_t kWaveMean = 64;
+bool wave_route(uint64_t n, uint64_t num_segments, bool value_order) {
+    return !value_order && num_segments <= n / kWaveMean;
+}
+
 template <typename K, typename V, bool PAIRS, int KIND>
 int segsort(K* keys_in, K* keys_out, K* keys_scratch, V* values_in, V* values_out, V* values_scratch, uint64_t n,
             uint64_t num_segments, const uint32_t* begins, const uint32_t* ends, uint32_t begin_bit, uint32_t end_bit,
@@ -931,7 +940,15 @@ int segsort(K* keys_in, K* keys_out, K* keys_scratch, V* values_in, V* values_ou
     }
     const uint64_t tiles = ceil_div(n, kSsChunk);
     const uint64_t cap = static_cast<uint64_t>(device_cu_count()) * 8;
-    {
+    const uint64_t tile_cap = cap * 4;
+    const unsigned tile_grid = static_cast<unsigned>(tiles < tile_cap ? tiles : tile_cap);
+    if (wave_route(n, num_segments, o.value_order)) {
+        const SegmentKeys kind = KIND == kKindFloat ? SegmentKeys::kFloat
+                                 : KIND == kKindSigned ? SegmentKeys::kSigned : SegmentKeys::kUnsigned;
+        st = segsort_waves<K, V, PAIRS>(keys_in, keys_out, values_in, values_out, begins, ends, num_segments, n, kind,
+                                        begin_bit, end_bit, descending != 0, words, stream);
+        if (st != kOk) return st;
+    } else {
         // About one workgroup per 4,096 items (groups of segment offsets: with tiny and small segments each
         // workgroup reads many), but at least 8 per CU where the input allows, and never more than n / kSsSmall
         // (the most segments that can be medium).  Measured on 2^26 u32 keys against one per 512 items:
@@ -941,27 +958,27 @@ int segsort(K* keys_in, K* keys_out, K* keys_scratch, V* values_in, V* values_ou
         const uint64_t target = n / (8 * kSsSmall) > fill ? n / (8 * kSsSmall) : fill;
         const uint64_t per_group = ceil_div(num_segments, target);
         const unsigned groups = static_cast<unsigned>(ceil_div(num_segments, per_group));
-        LaunchScope scope("segsort_block", stream);
-        segsort_block_kernel<K, V, PAIRS, KIND><<<groups, kSsBlock, 0, stream>>>(
-            keys_in, keys_out, values_in, values_out, begins, ends, static_cast<uint32_t>(num_segments),
-            static_cast<uint32_t>(per_group), n, o, words);
-        st = check_hip(hipGetLastError(), "segsort block launch");
-        if (st != kOk) return st;
-    }
-    {
+        {
+            LaunchScope scope("segsort_block", stream);
+            segsort_block_kernel<K, V, PAIRS, KIND><<<groups, kSsBlock, 0, stream>>>(
+                keys_in, keys_out, values_in, values_out, begins, ends, static_cast<uint32_t>(num_segments),
+                static_cast<uint32_t>(per_group), n, o, words);
+            st = check_hip(hipGetLastError(), "segsort block launch");
+            if (st != kOk) return st;
+        }
         // Tile and chunk kernels: grid-stride over 2,048-item tiles with enough workgroups to hide each
         // tile's segment searches; with no small (long) segment they exit after one word read.
-        const uint64_t tile_cap = cap * 4;
-        const unsigned tile_grid = static_cast<unsigned>(tiles < tile_cap ? tiles : tile_cap);
         LaunchScope scope("segsort_tile", stream);
         segsort_tile_kernel<K, V, PAIRS, KIND><<<tile_grid, kSsBlock, 0, stream>>>(
             keys_in, keys_out, keys_scratch, values_in, values_out, values_scratch, begins, ends,
             static_cast<uint32_t>(num_segments), n, o, words);
         st = check_hip(hipGetLastError(), "segsort tile launch");
         if (st != kOk) return st;
+    }
+    {
         const uint32_t chunk = o.value_order ? kSsChunk : kSsRadixChunk;
         if (n <= chunk) return kOk;
-        LaunchScope scope2("segsort_chunk", stream);
+        LaunchScope scope("segsort_chunk", stream);
         segsort_chunk_kernel<K, V, PAIRS, KIND><<<tile_grid, kSsBlock, 0, stream>>>(
             keys_in, keys_out, keys_scratch, values_in, values_out, values_scratch, begins, ends,
             static_cast<uint32_t>(num_segments), n, o, words);

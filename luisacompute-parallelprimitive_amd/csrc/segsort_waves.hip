@@ -1,0 +1,271 @@
+// Segmented radix-order sort of every segment that fits LDS, for gfx950: a wave per small segment and a
+// workgroup per medium one, in one launch.
+//
+// The other route (segsort.hip) sorts small segments jointly per 2,048-item tile, which costs a pass over their
+// labels, a second sort of the segment that crosses the tile's end and two searches per tile, in a launch of its
+// own; its chain of LDS round trips and barriers runs 4 items per lane and pass at 16 waves per CU (78 us at 4 M
+// u32 + u32 pairs in 13,333 log-normal segments of mean 300, and 73 us more for the medium segments).  Here:
+//   * A wave sorts up to 512 items with no barrier: digits are ranked by ballot matches against the wave's own
+//     256 counters, four of which each lane scans, and the items move through the wave's own LDS.  Items per
+//     lane follow the length (1, 2, 4 or 8), since a rank step costs the same whether its items are real.
+//   * Medium segments are collected by the workgroup's waves and sorted by all 512 threads, 2, 4 or 8 items per
+//     thread.
+//   * Digits that are the same in a whole segment are skipped.
+// The kinds of key differ by two mask words, so the code exists once per key and value size.
+#include "block_sort.hpp"
+#include "segsort_waves.hpp"
+
+#include <algorithm>
+
+namespace lcpp_hip {
+namespace {
+
+constexpr int kSwBlock = 512;
+constexpr int kSwWaves = kSwBlock / kWave;
+constexpr uint32_t kSwSmall = 512;    // items that one wave sorts
+constexpr uint32_t kSwMedium = 4096;  // items that the workgroup sorts
+constexpr uint32_t kSwPerWave = kSwMedium / kSwWaves;
+static_assert(kSwSmall <= kSwPerWave, "a wave's share of the workgroup's arrays holds a small segment");
+
+// Compared bits of a key, in the low bits of a word.
+template <typename U>
+struct SegmentBits {
+    U float_mask, sign_mask, desc_mask, bit_mask;
+    uint32_t begin;
+    __device__ __forceinline__ U operator()(U x) const {
+        const U all = static_cast<U>(static_cast<std::make_signed_t<U>>(x) >> (sizeof(U) * 8 - 1));
+        return ((x ^ ((all & float_mask) | sign_mask) ^ desc_mask) >> begin) & bit_mask;
+    }
+};
+
+// One wave's view of the workgroup's LDS.
+template <typename U, typename V, bool PAIRS>
+struct WaveLds {
+    U* key;
+    V* value;
+    uint32_t* count;  // 256, 16-byte aligned
+};
+
+// LDS written by a lane is read by others of its wave: in order in hardware; this keeps the compiler to it.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+struct OrOp {
+    template <typename T>
+    __device__ __forceinline__ T operator()(T a, T b) const { return a | b; }
+    template <typename T>
+    __device__ __forceinline__ static constexpr T identity() { return T(0); }
+};
+
+// Stable sort of the segment [at, at + len), len <= 64 ITEMS, by one wave; every item is read before any is
+// written.  Item j of lane l is item 64 j + l.
+template <typename U, typename V, bool PAIRS, int ITEMS>
+__device__ __forceinline__ void wave_sort(const U* keys_in, U* keys_out, const V* values_in, V* values_out, uint64_t at,
+                                          uint32_t len, uint32_t bits, const SegmentBits<U>& sort_bits,
+                                          const WaveLds<U, V, PAIRS>& s) {
+    typedef uint32_t Four __attribute__((ext_vector_type(4)));
+    const uint32_t lane = lane_id();
+    U k[ITEMS];
+    V v[PAIRS ? ITEMS : 1];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t i = j * kWave + lane;
+        k[j] = i < len ? keys_in[at + i] : U(0);
+        if constexpr (PAIRS) v[j] = i < len ? values_in[at + i] : V(0);
+    }
+    const U ref = wave_read_lane(sort_bits(k[0]), 0);
+    U vary = 0;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+        if (j * kWave + lane < len) vary |= sort_bits(k[j]) ^ ref;
+    vary = wave_reduce(vary, OrOp{});
+    Four* const quads = reinterpret_cast<Four*>(s.count);
+    for (uint32_t shift = 0; shift < bits; shift += 8) {
+        if ((static_cast<uint32_t>(vary >> shift) & 0xFFu) == 0) continue;
+        quads[lane] = Four{0u, 0u, 0u, 0u};
+        wave_lds_order();
+        uint32_t rank[ITEMS];  // digit << 16 | rank among the items of that digit
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            uint32_t d = static_cast<uint32_t>(sort_bits(k[j]) >> shift) & 0xFFu;
+            if (j * kWave + lane >= len) d = 0xFFu;  // missing items rank last
+            const uint64_t peers = match_digit(d);
+            const uint32_t below = popc_lanes_below(peers);
+            const uint32_t base = s.count[d];
+            rank[j] = (d << 16) | (base + below);
+            if ((peers >> lane) == 1ull) s.count[d] = base + below + 1;
+            wave_lds_order();
+        }
+        Four c = quads[lane];
+        const uint32_t sum = c[0] + c[1] + c[2] + c[3];
+        uint32_t start = wave_inclusive_scan(sum, SumOp{}) - sum;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t n = c[i];
+            c[i] = start;
+            start += n;
+        }
+        quads[lane] = c;
+        wave_lds_order();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const uint32_t pos = s.count[rank[j] >> 16] + (rank[j] & 0xFFFFu);
+            s.key[pos] = k[j];
+            if constexpr (PAIRS) s.value[pos] = v[j];
+        }
+        wave_lds_order();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            k[j] = s.key[j * kWave + lane];
+            if constexpr (PAIRS) v[j] = s.value[j * kWave + lane];
+        }
+        wave_lds_order();
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t i = j * kWave + lane;
+        if (i < len) {
+            keys_out[at + i] = k[j];
+            if constexpr (PAIRS) values_out[at + i] = v[j];
+        }
+    }
+}
+
+template <typename U, typename V, bool PAIRS, int ITEMS>
+__device__ __forceinline__ void block_sort_segment(const U* keys_in, U* keys_out, const V* values_in, V* values_out,
+                                                   uint64_t at, uint32_t len, uint32_t bits,
+                                                   const SegmentBits<U>& sort_bits, unsigned char* lds) {
+    using Sorter = BlockSort<U, V, PAIRS, kSwBlock, ITEMS>;
+    const uint32_t first = threadIdx.x / kWave * kWave * ITEMS + lane_id();
+    U k[ITEMS];
+    V v[PAIRS ? ITEMS : 1];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t i = first + j * kWave;
+        k[j] = i < len ? keys_in[at + i] : U(0);
+        if constexpr (PAIRS) v[j] = i < len ? values_in[at + i] : V(0);
+    }
+    Sorter::sort(k, v, len, bits, sort_bits, *reinterpret_cast<typename Sorter::Shared*>(lds));
+    __syncthreads();  // every item is read, and the LDS is free for the next segment
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t i = first + j * kWave;
+        if (i < len) {
+            keys_out[at + i] = k[j];
+            if constexpr (PAIRS) values_out[at + i] = v[j];
+        }
+    }
+}
+
+// Workgroup g takes the segments [g * per_group, (g + 1) * per_group), each wave per_wave (<= 64) of them, whose
+// bounds its lanes read together.  The longest segment above kSwMedium goes to words[0] (a load first:
+// atomics on one address serialise).
+// 40 KB of LDS for four-byte pairs: three workgroups per CU, 24 waves, at most 80 VGPRs.
+template <typename U, typename V, bool PAIRS>
+__global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 ? 6 : 4) void segsort_waves_kernel(
+    const U* keys_in, U* keys_out, const V* values_in, V* values_out, const uint32_t* __restrict__ begins,
+    const uint32_t* __restrict__ ends, uint32_t num_segments, uint32_t per_group, uint32_t per_wave, uint64_t n, uint32_t bits,
+    SegmentBits<U> sort_bits, uint32_t* words) {
+    using Sorter = BlockSort<U, V, PAIRS, kSwBlock, static_cast<int>(kSwMedium / kSwBlock)>;
+    static_assert(sizeof(U) * kSwSmall + (PAIRS ? sizeof(V) * kSwSmall : 0) + 1024 <= sizeof(typename Sorter::Shared) / kSwWaves,
+                  "the waves' arrays fit the workgroup's");
+    __shared__ __attribute__((aligned(16))) unsigned char s_lds[sizeof(typename Sorter::Shared)];
+    __shared__ uint16_t s_medium[kSwWaves * kWave];  // segments of the group, by number
+    __shared__ uint32_t s_mediums, s_long;
+    const uint32_t lane = lane_id();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (threadIdx.x == 0) {
+        s_mediums = 0;
+        s_long = 0;
+    }
+    __syncthreads();
+    constexpr uint32_t kWaveBytes = 1024 + kSwSmall * (sizeof(U) + (PAIRS ? sizeof(V) : 0));
+    unsigned char* const mine = s_lds + wave * kWaveBytes;
+    const WaveLds<U, V, PAIRS> s{reinterpret_cast<U*>(mine + 1024), reinterpret_cast<V*>(mine + 1024 + kSwSmall * sizeof(U)),
+                                 reinterpret_cast<uint32_t*>(mine)};
+    const uint64_t group = static_cast<uint64_t>(blockIdx.x) * per_group;
+    const uint32_t member = wave * per_wave + lane;
+    const uint64_t x = group + member;
+    uint32_t b = 0, len = 0;
+    if (lane < per_wave && member < per_group && x < num_segments) {
+        b = begins[x];
+        const uint32_t e = ends[x];
+        len = b < e && e <= n ? e - b : 0u;
+    }
+    if (len > kSwMedium) {
+        atomicMax(&s_long, len);
+    } else if (len > kSwSmall) {
+        s_medium[atomicAdd(&s_mediums, 1u)] = static_cast<uint16_t>(member);
+    } else if (len == 1) {
+        keys_out[b] = keys_in[b];
+        if constexpr (PAIRS) values_out[b] = values_in[b];
+    }
+    uint64_t small = wave_ballot(len > 1 && len <= kSwSmall);
+    while (small != 0) {
+        const uint32_t from = static_cast<uint32_t>(__builtin_ctzll(small));
+        small &= small - 1;
+        const uint64_t at = __builtin_amdgcn_readlane(b, from);
+        const uint32_t l = __builtin_amdgcn_readlane(len, from);
+        if (l <= 64) wave_sort<U, V, PAIRS, 1>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
+        else if (l <= 128) wave_sort<U, V, PAIRS, 2>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
+        else if (l <= 256) wave_sort<U, V, PAIRS, 4>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
+        else wave_sort<U, V, PAIRS, 8>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
+    }
+    __syncthreads();  // the list is complete, and the waves are done with their LDS
+    const uint32_t mediums = s_mediums;
+    for (uint32_t i = 0; i < mediums; ++i) {
+        const uint64_t y = group + s_medium[i];
+        const uint64_t at = begins[y];
+        const uint32_t l = ends[y] - static_cast<uint32_t>(at);
+        if (l <= 1024) block_sort_segment<U, V, PAIRS, 2>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s_lds);
+        else if (l <= 2048) block_sort_segment<U, V, PAIRS, 4>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s_lds);
+        else block_sort_segment<U, V, PAIRS, 8>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s_lds);
+    }
+    if (words && threadIdx.x == 0 && s_long &&
+        __hip_atomic_load(&words[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < s_long)
+        atomicMax(&words[0], s_long);
+}
+
+}  // namespace
+
+template <typename U, typename V, bool PAIRS>
+int segsort_waves(const U* keys_in, U* keys_out, const V* values_in, V* values_out, const uint32_t* begins,
+                  const uint32_t* ends, uint64_t num_segments, uint64_t n, SegmentKeys kind, uint32_t begin_bit,
+                  uint32_t end_bit, bool descending, uint32_t* words, hipStream_t stream) {
+    const uint32_t bits = end_bit - begin_bit;
+    SegmentBits<U> sort_bits;
+    sort_bits.float_mask = kind == SegmentKeys::kFloat ? static_cast<U>(~U(0)) : U(0);
+    sort_bits.sign_mask = kind == SegmentKeys::kUnsigned ? U(0) : static_cast<U>(U(1) << (sizeof(U) * 8 - 1));
+    sort_bits.desc_mask = descending ? static_cast<U>(~U(0)) : U(0);
+    sort_bits.bit_mask = bits == 0 ? U(0) : static_cast<U>(static_cast<U>(~U(0)) >> (sizeof(U) * 8 - bits));
+    sort_bits.begin = bits == 0 ? 0u : begin_bit;
+    // Fewer than eight segments per workgroup while the workgroups do not fill the chip (three per CU): most of them
+    // may be medium, and those of a workgroup are sorted one after the other (33 segments of mean 1,500: 105.8 us per
+    // call with eight, 58.5 with one).  More than one per wave from four rounds of workgroups on, so that short
+    // segments cost a part of a workgroup's start.
+    const uint64_t resident = static_cast<uint64_t>(device_cu_count()) * 3;
+    const uint64_t per_wave = std::clamp<uint64_t>(num_segments / (resident * kSwWaves * 4), 1, kWave);
+    const uint64_t per_group =
+        per_wave > 1 ? per_wave * kSwWaves : std::clamp<uint64_t>(num_segments / resident, 1, kSwWaves);
+    const uint64_t groups = ceil_div(num_segments, per_group);
+    LaunchScope scope("segsort_waves", stream);
+    segsort_waves_kernel<U, V, PAIRS><<<static_cast<unsigned>(groups), kSwBlock, 0, stream>>>(
+        keys_in, keys_out, values_in, values_out, begins, ends, static_cast<uint32_t>(num_segments),
+        static_cast<uint32_t>(per_group), static_cast<uint32_t>(per_wave), n, bits, sort_bits, words);
+    return check_hip(hipGetLastError(), "segsort waves launch");
+}
+
+#define LCPP_HIP_SEGSORT_WAVES(U, V, P)                                                                            \
+    template int segsort_waves<U, V, P>(const U*, U*, const V*, V*, const uint32_t*, const uint32_t*, uint64_t,    \
+                                        uint64_t, SegmentKeys, uint32_t, uint32_t, bool, uint32_t*, hipStream_t);
+LCPP_HIP_SEGSORT_WAVES(uint32_t, uint32_t, false)
+LCPP_HIP_SEGSORT_WAVES(uint32_t, uint32_t, true)
+LCPP_HIP_SEGSORT_WAVES(uint32_t, uint64_t, true)
+LCPP_HIP_SEGSORT_WAVES(uint64_t, uint32_t, false)
+LCPP_HIP_SEGSORT_WAVES(uint64_t, uint32_t, true)
+LCPP_HIP_SEGSORT_WAVES(uint64_t, uint64_t, true)
+#undef LCPP_HIP_SEGSORT_WAVES
+
+}  // namespace lcpp_hip

@@ -1,0 +1,17 @@
+// segsort_waves (segsort_waves.hip): sorts every segment of up to 4,096 items in radix order.
+#pragma once
+
+#include "common.hpp"
+
+namespace lcpp_hip {
+
+enum class SegmentKeys { kUnsigned, kSigned, kFloat };
+
+// Stable; in place when the outputs are the inputs.  Longer segments are left alone, and the length of the
+// longest one is posted to words[0] when `words` is set.
+template <typename U, typename V, bool PAIRS>
+int segsort_waves(const U* keys_in, U* keys_out, const V* values_in, V* values_out, const uint32_t* begins,
+                  const uint32_t* ends, uint64_t num_segments, uint64_t n, SegmentKeys kind, uint32_t begin_bit,
+                  uint32_t end_bit, bool descending, uint32_t* words, hipStream_t stream);
+
+}  // namespace lcpp_hip

@@ -1,0 +1,73 @@
+"""Segmented radix-order sorts whose segments average 64 items or more: a wave or a workgroup per segment.
+Lengths at the edges of the items per lane (64, 128, 256, 512) and per thread (1,024, 2,048, 4,096), empty
+segments, gaps that stay untouched, partial bit ranges and several segments per wave, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import to_dev, to_host
+from test_gpu_segsort import NP, check, g_sort
+
+pytestmark = pytest.mark.gpu
+EDGES = [0, 1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097,
+         9000]
+
+
+def words(rng, n, ks):
+    k = rng.integers(0, 1 << 64, n, dtype=np.uint64).view(np.uint8)[:n * np.dtype(NP[ks]).itemsize].view(NP[ks]).copy()
+    if ks in ("f32", "f64"):
+        k = np.where(np.isfinite(k), k, NP[ks](0))
+        k[::5] = NP[ks](-0.0)
+    else:
+        k[::3] &= NP[ks](0x70F)
+    return k
+
+
+def layout(rng, lengths):
+    """Segments in random order, some behind a gap."""
+    lengths = rng.permutation(lengths)
+    gaps = rng.integers(0, 2, lengths.size) * rng.integers(0, 40, lengths.size)
+    e = np.cumsum(lengths + gaps)
+    return (e - lengths).astype(np.uint32), e.astype(np.uint32), int(e[-1]) + 7
+
+
+@pytest.mark.parametrize("ks", ["u32", "i32", "f32", "u64", "i64", "f64"])
+@pytest.mark.parametrize("vb", [0, 4, 8])
+@pytest.mark.parametrize("desc", [False, True])
+def test_lengths_at_the_edges(hip, orc, dev, ks, vb, desc):
+    rng = np.random.default_rng(vb + desc)
+    b, e, n = layout(rng, np.array(EDGES + EDGES[:14]))
+    keys = words(rng, n, ks)
+    vals = np.arange(n, dtype=np.uint32 if vb == 4 else np.uint64) if vb else None
+    for begin, end in [(0, None), (3, 17), (5, 5)]:
+        kw = dict(begin_bit=begin, end_bit=end, descending=desc)
+        gk, gv = g_sort(hip, keys, b, e, values=vals, **kw)
+        kw["end_bit"] = 8 * keys.itemsize if end is None else end
+        check(orc, keys, b, e, gk, gv, values=vals, **kw)
+
+
+def test_several_segments_per_wave(hip, orc, dev):
+    rng = np.random.default_rng(3)
+    b, e, n = layout(rng, np.concatenate([rng.integers(0, 150, 110_000), [513, 1500, 4096, 4097, 5000]]))
+    assert len(b) <= n // 64
+    keys = words(rng, n, "u32")
+    vals = np.arange(n, dtype=np.uint32)
+    gk, gv = g_sort(hip, keys, b, e, values=vals)
+    check(orc, keys, b, e, gk, gv, values=vals)
+
+
+def test_double_buffer_in_place(hip, orc, dev):
+    """ceil(log2 n) is even: the result goes where the input is."""
+    rng = np.random.default_rng(4)
+    n = 60_000
+    b = np.arange(0, n, 1000, dtype=np.uint32)
+    e = np.minimum(b + rng.integers(0, 1001, b.size), n).astype(np.uint32)
+    b, e = b[:60], e[:60]
+    keys, vals = words(rng, n, "u32"), np.arange(n, dtype=np.uint32)
+    k0, v0 = to_dev(keys), to_dev(vals)
+    k1, v1 = torch.zeros_like(k0), torch.zeros_like(v0)
+    sel = hip.segmented_sort_db("u32", k0, k1, 0, n, b.size, to_dev(b), to_dev(e), values0=v0, values1=v1)
+    wk, wv = orc.segmented_sort(keys, b, e, values=vals, keys_out=keys.copy(), values_out=vals.copy())
+    assert sel == (0, 0)
+    np.testing.assert_array_equal(to_host(k0, np.uint32, n), wk)
+    np.testing.assert_array_equal(to_host(v0, np.uint32, n), wv)
