@@ -31,7 +31,7 @@
 //     (word 0 with release ordering where a helper and the owner could both write word 1), so the
 //     flag pair identifies one publication.
 // Algorithmic traffic: 2 * n * sizeof(T) bytes (read input, write output) + 8 * sizeof(T) / 4 bytes per tile.
-#include "common.hpp"
+#include "scan_small.hpp"
 #include "../../include/lcpp_hip.h"
 
 #include <limits>
@@ -423,12 +423,19 @@ int scan_op(const char* what, void* temp, size_t temp_bytes, const T* in, T* out
     if (reinterpret_cast<uintptr_t>(temp) % 8 != 0)
         return set_error(kInvalidArgument, "%s: temp storage must be 8-byte aligned", what);
 
+    const int vector_io = (reinterpret_cast<uintptr_t>(in) % 16 == 0) && (reinterpret_cast<uintptr_t>(out) % 16 == 0);
+    if constexpr (!std::is_same_v<Op, LeftOp>) {  // whose sentinel only the single-pass kernel knows
+        if (scan_small_route<T>(n, temp_bytes)) {
+            const char* name = std::is_same_v<Op, SumOp> ? "scan_sum" : "scan_minmax";
+            return inclusive ? scan_small<T, Op, true>(name, static_cast<T*>(temp), in, out, n, init, vector_io, stream)
+                             : scan_small<T, Op, false>(name, static_cast<T*>(temp), in, out, n, init, vector_io, stream);
+        }
+    }
     const uint64_t tiles = ceil_div(n, kScanTile<T>);
     uint64_t* states = static_cast<uint64_t*>(temp);
     int st = launch_fill_u32(static_cast<uint32_t*>(temp), needed / 4, 0u, stream);
     if (st != kOk) return st;
 
-    const int vector_io = (reinterpret_cast<uintptr_t>(in) % 16 == 0) && (reinterpret_cast<uintptr_t>(out) % 16 == 0);
     const uint32_t spin_limit = lookback_spin_limit();
     LaunchScope scope(std::is_same_v<Op, SumOp> ? "scan_sum" : std::is_same_v<Op, LeftOp> ? "scan_left" : "scan_minmax",
                       stream);
