@@ -223,6 +223,7 @@ struct CompactArgs {
     Predicate<P> pred;    // select / flagged-if / three-way first
     Predicate<P> pred2;   // three-way second
     uint32_t spin_limit;
+    uint32_t window;  // states per look-back step of the rows kernel
     bool partition;       // select: write the rejected items backwards after the selected ones
 };
 
@@ -749,8 +750,14 @@ constexpr int kRowItems = static_cast<int>(16 / sizeof(U));
 // 0.392 / 0.449 with 12 rows at five, 0.400 / 0.462 with 10 rows at six.
 template <typename U, bool FLAGS>
 constexpr int kSelRows = (FLAGS || sizeof(U) == 8) ? 12 : 16;
-template <typename U, bool FLAGS>
-constexpr uint32_t kRowsTile = static_cast<uint32_t>(kRowsBlock) * kSelRows<U, FLAGS> * kRowItems<U>;
+// Smaller inputs take smaller tiles, for enough of them to fill the chip, and a whole wave of states per look-back
+// step: their tiles run together and publish together, so a walk of short steps is a chain of round trips.
+// Select-if of u32, a third kept, per call with 16 rows and 8 states / 8 rows and 64 / 4 rows and 64:
+// 1,000,003 items 19.2 / 13.1 / 12.8 us, 4,000,037 22.6 / 15.5 / 13.7, 6,000,003 25.1 / 18.4 / 17.6, 10,000,019
+// 29.0 / 22.0 / 25.3, 40,000,003 73.8 / 63.5 / 78.6; partition of 64 M 113.8 / 122.4; 20 M u64 66.0 / 64.5 / 82.8.
+constexpr uint64_t kSel4Tiles = 1536, kSel8Tiles = 5120;
+template <typename U, int R>
+constexpr uint32_t kRowsTile = static_cast<uint32_t>(kRowsBlock) * R * kRowItems<U>;
 
 // One thread's items (and flags) of one row: items base + (256 r + tid) V + j, j < V, as one vector each.
 template <typename U, typename P>
@@ -806,11 +813,11 @@ __device__ __forceinline__ void load_row(const CompactArgs<U, P, U>& a, uint64_t
 
 // Selected items of tile `tile`, counted by one wave (a predecessor's count for the look-back fallback;
 // integer counts, so any order gives its owner's result).
-template <typename U, typename P, bool FLAGS>
+template <typename U, typename P, bool FLAGS, int R>
 __device__ uint32_t rows_tile_count(const CompactArgs<U, P, U>& a, uint32_t tile) {
     using RV = RowVecs<U, P>;
     constexpr int V = RV::V;
-    constexpr uint32_t TILE = kRowsTile<U, FLAGS>;
+    constexpr uint32_t TILE = kRowsTile<U, R>;
     const uint64_t base = static_cast<uint64_t>(tile) * TILE;
     const uint32_t lane = lane_id();
     uint32_t c = 0;
@@ -833,11 +840,11 @@ __device__ uint32_t rows_tile_count(const CompactArgs<U, P, U>& a, uint32_t tile
 }
 
 // Selected items before tile `tile` (> 0), by wave 0 alone (no workgroup barrier per poll): each step reads
-// kRowsWindow predecessor states, newest first, and sums them down to the nearest INCLUSIVE one.  A
+// a.window predecessor states, newest first, and sums them down to the nearest INCLUSIVE one.  A
 // predecessor still unpublished after `spin_limit` polls is claimed (claims[t]: OPEN -> HELPER), counted by
 // this wave and published PARTIAL, and its claim marked DONE with release ordering; a claim lost to the
 // owner or to another helper is simply polled again.
-template <typename U, typename P, bool FLAGS>
+template <typename U, typename P, bool FLAGS, int R>
 __device__ uint32_t rows_lookback(const CompactArgs<U, P, U>& a, uint64_t* states, uint64_t* claims, uint32_t tile) {
     const uint32_t lane = lane_id();
     uint32_t acc = 0;
@@ -845,7 +852,7 @@ __device__ uint32_t rows_lookback(const CompactArgs<U, P, U>& a, uint64_t* state
     uint32_t spins = 0;
     while (true) {
         const int64_t j = top - static_cast<int64_t>(lane);
-        const bool exists = j >= 0 && lane < static_cast<uint32_t>(kRowsWindow);
+        const bool exists = j >= 0 && lane < a.window;
         uint32_t v[1] = {0};
         const uint32_t st = exists ? read_words<1>(states + j, v) : kStInvalid;
         const bool published = st != kStInvalid;
@@ -869,7 +876,7 @@ __device__ uint32_t rows_lookback(const CompactArgs<U, P, U>& a, uint64_t* state
                           : 0u;
             }
             if (wave_read_lane(won, 0) != 0) {
-                const uint32_t h[1] = {rows_tile_count<U, P, FLAGS>(a, help_tile)};
+                const uint32_t h[1] = {rows_tile_count<U, P, FLAGS, R>(a, help_tile)};
                 if (lane == 0) {
                     publish_words<1>(states + help_tile, kStPartial, h);
                     __hip_atomic_store(&claims[help_tile], kClaimDone, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
@@ -879,19 +886,18 @@ __device__ uint32_t rows_lookback(const CompactArgs<U, P, U>& a, uint64_t* state
             continue;
         }
         acc += wave_reduce(exists && lane <= cut ? v[0] : 0u, SumOp{});
-        if (stop_mask != 0 || top < kRowsWindow) break;
-        top -= kRowsWindow;
+        if (stop_mask != 0 || top < static_cast<int64_t>(a.window)) break;
+        top -= a.window;
         spins = 0;
     }
     return acc;
 }
 
-template <typename U, typename P, bool FLAGS>
+template <typename U, typename P, bool FLAGS, int R>
 __global__ __launch_bounds__(kRowsBlock, 4) void select_rows_kernel(const CompactArgs<U, P, U> a) {
     using RV = RowVecs<U, P>;
     constexpr int V = RV::V;
-    constexpr int R = kSelRows<U, FLAGS>;
-    constexpr uint32_t TILE = kRowsTile<U, FLAGS>;
+    constexpr uint32_t TILE = kRowsTile<U, R>;
     constexpr int ROWS_PER_WORD = 32 / V;  // row masks packed into 32-bit words
     constexpr int MW = (R + ROWS_PER_WORD - 1) / ROWS_PER_WORD;
     constexpr uint32_t kRowSlots = static_cast<uint32_t>(kWave) * V;  // items of one wave's part of a row
@@ -985,7 +991,7 @@ __global__ __launch_bounds__(kRowsBlock, 4) void select_rows_kernel(const Compac
                         ? 1u
                         : 0u;
         }
-        if (tile > 0) prefix[0] = rows_lookback<U, P, FLAGS>(a, states, claims, tile);
+        if (tile > 0) prefix[0] = rows_lookback<U, P, FLAGS, R>(a, states, claims, tile);
         if (lane == 0) {
             if (!owned) {
                 while (__hip_atomic_load(&claims[tile], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) != kClaimDone)
@@ -1220,16 +1226,25 @@ int run_compact(const char* what, void* temp, size_t temp_bytes, const U* in, co
     if constexpr (MODE == kSelect && std::is_same_v<U, V> && (sizeof(U) == 4 || sizeof(U) == 8) &&
                   (!FLAGS || sizeof(P) <= 4)) {
         // Selects and partitions that are not in place take the register-resident rows kernel when the
-        // input (and the flags) allow whole-vector row loads.  Its tiles are larger, so its states take
-        // less temp storage than the plan checked above.
+        // input (and the flags) allow whole-vector row loads.  The states of its largest tiles take less temp
+        // storage than the plan checked above.
         if (!in_place && g_select_rows.load(std::memory_order_relaxed) && reinterpret_cast<uintptr_t>(in) % 16 == 0 &&
             (!FLAGS || reinterpret_cast<uintptr_t>(flags) % (kRowItems<U> * sizeof(P)) == 0)) {
-            const TempPlan rp = plan_temp(n, kRowsTile<U, FLAGS>, 1, 0);
-            int st = launch_fill_u32(reinterpret_cast<uint32_t*>(temp), rp.state_bytes / 4, 0u, stream);
-            if (st != kOk) return st;
-            LaunchScope scope("compact", stream);
-            select_rows_kernel<U, P, FLAGS><<<static_cast<unsigned>(rp.tiles), kRowsBlock, 0, stream>>>(a);
-            return check_hip(hipGetLastError(), "compact rows launch");
+            const auto launch = [&](auto rows, uint32_t window) {
+                constexpr int R = decltype(rows)::value;
+                const TempPlan rp = plan_temp(n, kRowsTile<U, R>, 1, 0);
+                a.window = window;
+                const int st = launch_fill_u32(reinterpret_cast<uint32_t*>(temp), rp.state_bytes / 4, 0u, stream);
+                if (st != kOk) return st;
+                LaunchScope scope("compact", stream);
+                select_rows_kernel<U, P, FLAGS, R><<<static_cast<unsigned>(rp.tiles), kRowsBlock, 0, stream>>>(a);
+                return check_hip(hipGetLastError(), "compact rows launch");
+            };
+            if (n <= static_cast<uint64_t>(kRowsTile<U, 4>) * kSel4Tiles && temp_bytes >= plan_temp(n, kRowsTile<U, 4>, 1, 0).total)
+                return launch(std::integral_constant<int, 4>{}, kWave);
+            if (n <= static_cast<uint64_t>(kRowsTile<U, 8>) * kSel8Tiles && temp_bytes >= plan_temp(n, kRowsTile<U, 8>, 1, 0).total)
+                return launch(std::integral_constant<int, 8>{}, kWave);
+            return launch(std::integral_constant<int, kSelRows<U, FLAGS>>{}, kRowsWindow);
         }
     }
     int st = launch_fill_u32(reinterpret_cast<uint32_t*>(temp), plan.state_bytes / 4, 0u, stream);

@@ -1,0 +1,85 @@
+"""Select, partition, by-key and run-length calls at the edges of the tiles they use for small and medium inputs
+and of the sizes where the tiles change, with and without the helped look-back, against numpy."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(params=[None, 0])
+def spin(hip, request):
+    lib = hip.lib()
+    old = lib.lcpp_hip_get_lookback_spin_limit()
+    if request.param is not None:
+        lib.lcpp_hip_set_lookback_spin_limit(request.param)
+    yield
+    lib.lcpp_hip_set_lookback_spin_limit(old)
+
+
+def around(*edges):
+    return [n + d for n in edges for d in (-1, 0, 1)]
+
+
+SELECT = [1, 63] + around(4096, 64 * 4096, 1536 * 4096, 5120 * 8192)
+
+
+@pytest.mark.parametrize("n", SELECT)
+def test_select_and_partition(hip, dev, spin, n):
+    x = np.random.default_rng(n).integers(0, 1 << 32, n, dtype=np.uint32)
+    d, num = to_dev(x), torch.zeros(1, dtype=torch.int32, device=dev)
+    keep = x < 0x55555555
+    for call in (hip.select_if, hip.partition_if):
+        out = torch.zeros_like(d)
+        call("u32", d, out, num, n, hip.predicate("u32", (hip.PRED_LT, 0x55555555)))
+        k = int(keep.sum())
+        assert int(num.item()) == k
+        got = out.cpu().numpy().view(np.uint32)
+        np.testing.assert_array_equal(got[:k], x[keep])
+        if call is hip.partition_if:
+            np.testing.assert_array_equal(got[k:], x[~keep][::-1])
+
+
+RUNS = [1, 3] + around(4096, 64 * 4096, (32 << 20) // 8, (24 << 20) // 4)
+
+
+@pytest.mark.parametrize("n", RUNS)
+@pytest.mark.parametrize("mean", [1, 9, 100_000])
+def test_runs_and_by_key(hip, dev, spin, n, mean):
+    rng = np.random.default_rng(n)
+    head = rng.random(n) < 1.0 / mean
+    head[0] = True
+    key = np.cumsum(head).astype(np.int32)
+    at = np.flatnonzero(head)
+    length = np.diff(np.append(at, n))
+    x = rng.integers(0, 1000, n).astype(np.int32)
+    dk, dx, num = to_dev(key), to_dev(x), torch.zeros(1, dtype=torch.int32, device=dev)
+    # 32-bit sums wrap: differences of a 64-bit running sum, reduced to 32 bits.
+    s = np.concatenate([[0], np.cumsum(x.astype(np.int64))])
+    for form in ("encode", "reduce"):
+        unique, second = torch.zeros_like(dk), torch.zeros_like(dk)
+        if form == "encode":
+            hip.run_length_encode("u32", dk, unique, second, num, n)
+            want = length
+        else:
+            hip.reduce_by_key("i32", "i32", dk, dx, unique, second, num, n)
+            want = s[at + length] - s[at]
+        assert int(num.item()) == at.size
+        np.testing.assert_array_equal(unique.cpu().numpy()[:at.size], key[at])
+        np.testing.assert_array_equal(second.cpu().numpy()[:at.size], want.astype(np.int32))
+    want = (s[:-1] - np.repeat(s[at], length)).astype(np.int32)
+    for out in (torch.zeros_like(dx), dx):  # the second in place
+        hip.scan_by_key("i32", "i32", dk, dx, out, n)
+        np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n", [42_000_000, 42_000_001])
+def test_scan_by_key_where_the_tiles_change(hip, dev, n):
+    x = np.random.default_rng(1).integers(0, 50, n).astype(np.int32)
+    key = (np.arange(n) // 1000).astype(np.int32)
+    out = torch.zeros(n, dtype=torch.int32, device=dev)
+    hip.scan_by_key("i32", "i32", to_dev(key), to_dev(x), out, n)
+    s = np.cumsum(x) - x
+    np.testing.assert_array_equal(out.cpu().numpy(), (s - s[::1000][key]).astype(np.int32))
