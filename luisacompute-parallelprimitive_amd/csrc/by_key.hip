@@ -19,7 +19,7 @@
 // MI355X design
 //   * Tile = 256 threads x R rows x 4 consecutive items per thread and row (R = 12 for 4-byte keys and
 //     values in the scan, 15 in the reduce, 22 in the count mode: 12,288 / 15,360 / 22,528 items; fewer
-//     for 8-byte types), every row a contiguous 1,024 items read (and, for the scan, written) with
+//     for 8-byte types, and 4 rows for smaller inputs), every row a contiguous 1,024 items read (and, for the scan, written) with
 //     16-byte vectors, all rows' loads in flight together; four workgroups per CU (three for the
 //     reduce).  The key before a thread-row is the previous
 //     lane's last key (DPP wave shift) or, for lane 0, the last key of the previous wave or row (a
@@ -37,7 +37,7 @@
 //     XCDs do not share an L2) and no fence is needed.  The owner publishes PARTIAL (tile 0:
 //     INCLUSIVE) with plain stores from lane 0 of its last wave: a wave's vector memory operations
 //     complete in issue order, so stores issued by wave 0 would delay its own look-back loads.
-//   * Look-back: wave 0 reads 32 predecessors per step (one per lane).  Ballots find the newest
+//   * Look-back: wave 0 reads up to 64 predecessors per step (one per lane).  Ballots find the newest
 //     INCLUSIVE state (or tile 0) and, for the scan, the newest state with a head: the scan stops
 //     there because older sums cannot reach this tile; ReduceByKey continues to an INCLUSIVE state
 //     since run indices need the full head count.  Counts and sums reduce with DPP.  Meanwhile the
@@ -105,6 +105,19 @@ constexpr int kBkRows =
 // Runs a reduce tile stages in LDS (32 KiB of keys and sums).
 template <typename K, typename V>
 constexpr uint32_t kBkStageItems = 32768u / static_cast<uint32_t>(sizeof(K) + sizeof(V));
+// Inputs of up to kBkSmallItems take tiles of 4 rows (4,096 items), enough of them to fill the chip.  Reduces and run
+// lengths, whose walk needs every earlier tile's count, read a whole wave of states per step there, since those
+// tiles run and publish together; a scan's walk mostly ends at the nearest head, and 8 states per step serve it up
+// to where its larger tiles stream as well.  Per call, full-size tiles -> 4 rows: ReduceByKey i32 / f32, runs of 20,
+// 1,000,003 items 15.3 -> 12.2 us, 4,000,037 19.3 -> 15.0, but 6,000,001 19.1 -> 20.9 (runs of 64; i64 / f64 2 M
+// 18.0 -> 16.9, 4 M 25.8 -> 30.0); encode u32, runs of 8, 1,000,003 18.9 -> 11.9, 4,000,037 21.4 -> 14.6, unique
+// 6,000,001 19.4 -> 18.5, encode 10,000,019 23.7 -> 29.1; ExclusiveSumByKey 1,000,003 15.7 -> 11.9, 4,000,037 18.4 ->
+// 12.7, 20,000,003 48.3 -> 44.9, 40,000,003 88.2 -> 82.8 (i64 / f64 6 M 39.7 -> 35.7).
+constexpr int kBkSmallRows = 4;
+template <typename K, typename V, int MODE>
+constexpr uint64_t kBkSmallItems = MODE == 0   ? 42'000'000
+                                   : MODE == 1 ? (32ull << 20) / (sizeof(K) + sizeof(V))
+                                               : (24ull << 20) / sizeof(K);
 template <typename K, typename V, int MODE>
 constexpr uint32_t kBkTileItems = static_cast<uint32_t>(kBkBlock * kBkVec * kBkRows<K, V, MODE>);
 
@@ -509,7 +522,7 @@ __global__ __launch_bounds__(kBkBlock, kBkBlocksPerCu<MODE>) void by_key_kernel(
     const K* __restrict__ keys, const V* values_in, V* values_out, K* __restrict__ unique_out,
     V* __restrict__ aggregates_out, uint32_t* __restrict__ num_runs_out, uint64_t n, K mask,
     uint64_t* __restrict__ states, int inclusive, int use_init, V init, bool vec_k, bool vec_v, bool vec_o,
-    bool in_place, uint32_t spin_limit) {
+    bool in_place, uint32_t spin_limit, uint32_t look_window) {
     constexpr bool COUNTED = MODE != kModeScan;
     constexpr int W = kStateWords<V, COUNTED>;
     uint64_t* const claims = states + static_cast<uint64_t>(gridDim.x) * W;
@@ -701,7 +714,7 @@ __global__ __launch_bounds__(kBkBlock, kBkBlocksPerCu<MODE>) void by_key_kernel(
             if (wave == 0) {
                 const int64_t j = top - static_cast<int64_t>(lane);
                 Seg<V> s{0u, op_identity<Op, V>()};
-                const bool exists = j >= 0 && lane < static_cast<uint32_t>(kBkWindow);
+                const bool exists = j >= 0 && lane < look_window;
                 const uint32_t st = exists ? read_state<V, COUNTED>(states + static_cast<uint64_t>(j) * W, s) : kStInvalid;
                 const bool published = st != kStInvalid;
                 // A complete prefix: an INCLUSIVE state, or tile 0 (nothing precedes it).
@@ -733,7 +746,7 @@ __global__ __launch_bounds__(kBkBlock, kBkBlocksPerCu<MODE>) void by_key_kernel(
                     acc = seg_combine<Op>(window, acc);
                     const bool complete = stop_mask != 0 && cut == static_cast<uint32_t>(__builtin_ctzll(stop_mask));
                     const bool found_head = MODE == kModeScan && heads_in != 0;
-                    action = (complete || found_head || top < kBkWindow) ? kActDone : kActAdvance;
+                    action = (complete || found_head || top < static_cast<int64_t>(look_window)) ? kActDone : kActAdvance;
                 }
                 if (lane == 0) {
                     s_ctl[row][0] = action;
@@ -747,7 +760,7 @@ __global__ __launch_bounds__(kBkBlock, kBkBlocksPerCu<MODE>) void by_key_kernel(
             row ^= 1u;
             if (action == kActDone) break;
             if (action == kActAdvance) {
-                top -= kBkWindow;
+                top -= look_window;
                 spins = 0;
                 continue;
             }
@@ -871,21 +884,30 @@ int by_key(void* temp, size_t temp_bytes, const K* keys, const V* values_in, V* 
                 if (ranges_overlap(outs[o], out_bytes[o], ins[i], in_bytes[i]))
                     return set_error(kInvalidArgument, "%s: outputs must not overlap the inputs", what);
     }
-    constexpr uint32_t kTile = kBkTileItems<K, V, MODE>;
-    const size_t need = state_bytes(n, kTile, sizeof(V), MODE != kModeScan);
+    constexpr int kRows = kBkRows<K, V, MODE>;
+    const size_t need = state_bytes(n, kBkTileItems<K, V, MODE>, sizeof(V), MODE != kModeScan);
     if (!temp || temp_bytes < need)
         return set_error(kTempTooSmall, "%s: temp storage too small (%zu < %zu bytes)", what, temp_bytes, need);
     if (reinterpret_cast<uintptr_t>(temp) % 8 != 0) return set_error(kInvalidArgument, "%s: temp not 8-byte aligned", what);
-    uint64_t* states = static_cast<uint64_t*>(temp);
-    int st = launch_fill_u32(reinterpret_cast<uint32_t*>(states), need / 4, 0u, stream);
-    if (st != kOk) return st;
-    const uint32_t tiles = static_cast<uint32_t>(ceil_div(n, kTile));
-    LaunchScope scope(MODE == kModeScan ? "scan_by_key" : MODE == kModeReduce ? "reduce_by_key" : "runs_by_key", stream);
-    by_key_kernel<K, V, MODE, kBkRows<K, V, MODE>, Op><<<tiles, kBkBlock, 0, stream>>>(
-        keys, values_in, values_out, unique_out, aggregates_out, num_runs_out, n, static_cast<K>(key_mask), states,
-        inclusive, use_init, init, aligned16(keys), aligned16(values_in), values_out != nullptr && aligned16(values_out),
-        values_out != nullptr && values_out == values_in, lookback_spin_limit());
-    return check_hip(hipGetLastError(), MODE == kModeScan ? "scan_by_key launch" : "reduce_by_key launch");
+    const auto launch = [&](auto rows, uint32_t window) {
+        constexpr int R = decltype(rows)::value;
+        constexpr uint32_t kTile = static_cast<uint32_t>(kBkBlock * kBkVec * R);
+        uint64_t* states = static_cast<uint64_t*>(temp);
+        const size_t bytes = state_bytes(n, kTile, sizeof(V), MODE != kModeScan);
+        const int st = launch_fill_u32(reinterpret_cast<uint32_t*>(states), bytes / 4, 0u, stream);
+        if (st != kOk) return st;
+        const uint32_t tiles = static_cast<uint32_t>(ceil_div(n, kTile));
+        LaunchScope scope(MODE == kModeScan ? "scan_by_key" : MODE == kModeReduce ? "reduce_by_key" : "runs_by_key", stream);
+        by_key_kernel<K, V, MODE, R, Op><<<tiles, kBkBlock, 0, stream>>>(
+            keys, values_in, values_out, unique_out, aggregates_out, num_runs_out, n, static_cast<K>(key_mask), states,
+            inclusive, use_init, init, aligned16(keys), aligned16(values_in), values_out != nullptr && aligned16(values_out),
+            values_out != nullptr && values_out == values_in, lookback_spin_limit(), window);
+        return check_hip(hipGetLastError(), MODE == kModeScan ? "scan_by_key launch" : "reduce_by_key launch");
+    };
+    if (n <= kBkSmallItems<K, V, MODE> &&
+        temp_bytes >= state_bytes(n, kBkBlock * kBkVec * kBkSmallRows, sizeof(V), MODE != kModeScan))
+        return launch(std::integral_constant<int, kBkSmallRows>{}, MODE == kModeScan ? 8u : static_cast<uint32_t>(kWave));
+    return launch(std::integral_constant<int, kRows>{}, static_cast<uint32_t>(kBkWindow));
 }
 
 }  // namespace
