@@ -932,8 +932,9 @@ __global__ __launch_bounds__(kRowsBlock, 4) void select_rows_kernel(const Compac
 #pragma unroll
                 for (int r = 0; r < R; ++r) fl[r] = __builtin_nontemporal_load(&fsrc[r * kRowsBlock + tid]);
             }
+            // The last word may hold fewer than 32 items; a clause that is always true sets its other bits too.
 #pragma unroll
-            for (int w = 0; w < MW; ++w) valid[w] = ~0u;
+            for (int w = 0; w < MW; ++w) valid[w] = (w + 1) * 32 <= R * V ? ~0u : (1u << (R * V % 32)) - 1u;
         } else {
 #pragma unroll
             for (int r = 0; r < R; ++r) {

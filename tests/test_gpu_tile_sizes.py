@@ -42,6 +42,20 @@ def test_select_and_partition(hip, dev, spin, n):
             np.testing.assert_array_equal(got[k:], x[~keep][::-1])
 
 
+@pytest.mark.parametrize("t", ["u32", "u64"])
+@pytest.mark.parametrize("n", [3 * 4096 + 5, 1536 * 4096 + 4097, 5120 * 8192 + 1])
+def test_select_everything(hip, dev, t, n):
+    """Rows whose masks fill a word only in part (4 rows of u32, every row count of u64)."""
+    np_t = np.uint32 if t == "u32" else np.uint64
+    x = np.random.default_rng(n).integers(0, 1 << 31, n).astype(np_t)
+    d, num = to_dev(x), torch.zeros(1, dtype=torch.int32, device=dev)
+    out = torch.zeros(2 * n, dtype=d.dtype, device=dev)  # room for a count twice too large
+    hip.select_if(t, d, out[:n], num, n, hip.predicate(t, (hip.PRED_TRUE,)))
+    assert int(num.item()) == n
+    np.testing.assert_array_equal(out.cpu().numpy().view(np_t)[:n], x)
+    assert not out[n:].any()
+
+
 RUNS = [1, 3] + around(4096, 64 * 4096, (32 << 20) // 8, (24 << 20) // 4)
 
 
