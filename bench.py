@@ -208,13 +208,13 @@ def extra_reduce(hip, dev, steps, warmup, extra):
     call = lambda: hip.reduce_sum("i32", a, s, m, temp=rt)
     # Per call from the host (one event per step: Python and launch gaps included), per call inside a
     # HIP graph of 20 calls (device time only), the whole call after a MALL flush, and the floor of the
-    # call's shape: the same two launches (partials + final fold) over 8,192 items, in a graph.
+    # call's shape: the same two launches (partials + final fold) over 20,000 items, in a graph.
     hot = time_steps(call, steps, warmup)
     hot_graph = graph_call_ms(call, 20, 10)
     cold = cold_call_ms(call, flush, 10)
-    tiny = torch.empty(8192, dtype=torch.int32, device=dev)
-    hip.generate(hip.GEN_I32_PM1000, tiny, 8192, SEED)
-    floor = graph_call_ms(lambda: hip.reduce_sum("i32", tiny, s, 8192, temp=rt), 20, 10)
+    tiny = torch.empty(20_000, dtype=torch.int32, device=dev)
+    hip.generate(hip.GEN_I32_PM1000, tiny, 20_000, SEED)
+    floor = graph_call_ms(lambda: hip.reduce_sum("i32", tiny, s, 20_000, temp=rt), 20, 10)
     extra["reduce_sum_i32_2p24"] = {**hot.fields("ms_hot"), "GBps_hot": rate(4 * m, hot.mean),
                                     **hot_graph.fields("ms_hot_graph"), "GBps_hot_graph": rate(4 * m, hot_graph.mean),
                                     **cold.fields("ms_cold"), "GBps_cold": rate(4 * m, cold.mean),

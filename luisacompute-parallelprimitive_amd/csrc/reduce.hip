@@ -9,7 +9,7 @@
 // 4,096 items) streams the input with 128-bit loads, UNROLL loads in flight per thread, folds them in registers,
 // reduces each wave with DPP row shifts / row broadcasts, and writes one partial per workgroup into
 // the caller's temp storage.  A single 1024-thread workgroup folds the partials and writes *out.
-// Inputs of at most one persistent round fall back to one workgroup that writes *out directly.
+// Inputs of at most 64 KB take one workgroup that writes *out directly.
 // Min and max run the same pass with the NaN-ignoring operators (reference MinOp / MaxOp, folded from
 // the type's max / lowest as the reference's initial value, device_reduce.h:291-309).  ArgMin / ArgMax
 // (device_reduce.h:311-436) fold (value, index) pairs: the smaller (larger) value wins, equal values the
@@ -33,9 +33,15 @@ constexpr int kFinalBlock = 1024;
 template <typename T>
 using Vec16 = T __attribute__((ext_vector_type(16 / sizeof(T))));
 
-template <typename T>
+// Inputs of up to one round of a 1,024-thread workgroup (64 KB) are folded by that workgroup alone: the second
+// launch costs more than the CUs it leaves idle (5,003 f32 9.8 -> 7.9 us per call, 16,384
+// 10.3 -> 7.8).
+constexpr int kOneBlock = 1024;
+constexpr uint64_t kOneBlockVecs = static_cast<uint64_t>(kOneBlock) * kReduceUnroll;
+
+template <int BLOCK, typename T>
 __device__ __forceinline__ T block_sum(T x, T* s_waves) {
-    constexpr int W = kReduceBlock / kWave;
+    constexpr int W = BLOCK / kWave;
     x = wave_reduce(x, SumOp{});
     const int wave = threadIdx.x / kWave;
     if (lane_id() == 0) s_waves[wave] = x;
@@ -48,13 +54,13 @@ __device__ __forceinline__ T block_sum(T x, T* s_waves) {
 
 // Folds in[0..n) into partials[blockIdx.x].  `head` leading elements precede the first 16-byte
 // aligned address; `nvec` aligned vectors follow; the remaining tail elements end the range.
-template <typename T>
-__global__ __launch_bounds__(kReduceBlock) void reduce_sum_partials_kernel(const T* __restrict__ in, uint64_t n,
+template <typename T, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void reduce_sum_partials_kernel(const T* __restrict__ in, uint64_t n,
                                                                            uint32_t head, uint64_t nvec,
                                                                            T* __restrict__ partials) {
     constexpr int V = 16 / sizeof(T);
     using Vec = Vec16<T>;
-    __shared__ T s_waves[kReduceBlock / kWave];
+    __shared__ T s_waves[BLOCK / kWave];
     const Vec* __restrict__ vin = reinterpret_cast<const Vec*>(in + head);
     const uint32_t tid = threadIdx.x;
 
@@ -62,13 +68,13 @@ __global__ __launch_bounds__(kReduceBlock) void reduce_sum_partials_kernel(const
 #pragma unroll
     for (int u = 0; u < kReduceUnroll; ++u) acc[u] = T(0);
 
-    const uint64_t chunk = static_cast<uint64_t>(kReduceBlock) * kReduceUnroll;
+    const uint64_t chunk = static_cast<uint64_t>(BLOCK) * kReduceUnroll;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * chunk;
     uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunk;
     for (; base + chunk <= nvec; base += stride) {
         Vec v[kReduceUnroll];
 #pragma unroll
-        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * kReduceBlock + tid]);
+        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * BLOCK + tid]);
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
             T s = v[u][0];
@@ -80,7 +86,7 @@ __global__ __launch_bounds__(kReduceBlock) void reduce_sum_partials_kernel(const
     if (base < nvec) {  // last, partial chunk of this workgroup
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
-            const uint64_t idx = base + u * kReduceBlock + tid;
+            const uint64_t idx = base + u * BLOCK + tid;
             if (idx < nvec) {
                 Vec v = vin[idx];
                 T s = v[0];
@@ -98,7 +104,7 @@ __global__ __launch_bounds__(kReduceBlock) void reduce_sum_partials_kernel(const
     T x = acc[0];
 #pragma unroll
     for (int u = 1; u < kReduceUnroll; ++u) x += acc[u];
-    x = block_sum(x, s_waves);
+    x = block_sum<BLOCK>(x, s_waves);
     if (tid == 0) partials[blockIdx.x] = x;
 }
 
@@ -169,9 +175,9 @@ struct WrapSumOp {
 };
 
 // ---- min / max ---------------------------------------------------------------------------------
-template <typename T, typename Op>
+template <int BLOCK, typename T, typename Op>
 __device__ __forceinline__ T block_fold(T x, T* s_waves, Op op) {
-    constexpr int W = kReduceBlock / kWave;
+    constexpr int W = BLOCK / kWave;
     x = wave_reduce(x, op);
     const int wave = threadIdx.x / kWave;
     if (lane_id() == 0) s_waves[wave] = x;
@@ -183,28 +189,29 @@ __device__ __forceinline__ T block_fold(T x, T* s_waves, Op op) {
 }
 
 // reduce_sum_partials_kernel with another operator (min / max, or the sum in the item's own type) and a
-// transform of every item; partials[blockIdx.x] = the workgroup's fold.
-template <typename T, typename Op, int XF = kXformIdentity>
-__global__ __launch_bounds__(kReduceBlock) void reduce_ext_partials_kernel(const T* __restrict__ in, uint64_t n,
+// transform of every item; partials[blockIdx.x] = the workgroup's fold, behind the
+// initial value when it is the only one.
+template <typename T, typename Op, int XF, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void reduce_ext_partials_kernel(const T* __restrict__ in, uint64_t n,
                                                                            uint32_t head, uint64_t nvec,
                                                                            T* __restrict__ partials, T scale,
-                                                                           T shift) {
+                                                                           T shift, T init) {
     constexpr int V = 16 / sizeof(T);
     using Vec = Vec16<T>;
     const Op op{};
-    __shared__ T s_waves[kReduceBlock / kWave];
+    __shared__ T s_waves[BLOCK / kWave];
     const Vec* __restrict__ vin = reinterpret_cast<const Vec*>(in + head);
     const uint32_t tid = threadIdx.x;
     T acc[kReduceUnroll];
 #pragma unroll
     for (int u = 0; u < kReduceUnroll; ++u) acc[u] = Op::template identity<T>();
-    const uint64_t chunk = static_cast<uint64_t>(kReduceBlock) * kReduceUnroll;
+    const uint64_t chunk = static_cast<uint64_t>(BLOCK) * kReduceUnroll;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * chunk;
     uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunk;
     for (; base + chunk <= nvec; base += stride) {
         Vec v[kReduceUnroll];
 #pragma unroll
-        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * kReduceBlock + tid]);
+        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * BLOCK + tid]);
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
 #pragma unroll
@@ -214,7 +221,7 @@ __global__ __launch_bounds__(kReduceBlock) void reduce_ext_partials_kernel(const
     if (base < nvec) {
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
-            const uint64_t idx = base + u * kReduceBlock + tid;
+            const uint64_t idx = base + u * BLOCK + tid;
             if (idx < nvec) {
                 const Vec v = vin[idx];
 #pragma unroll
@@ -230,8 +237,8 @@ __global__ __launch_bounds__(kReduceBlock) void reduce_ext_partials_kernel(const
     T x = acc[0];
 #pragma unroll
     for (int u = 1; u < kReduceUnroll; ++u) x = op(x, acc[u]);
-    x = block_fold(x, s_waves, op);
-    if (tid == 0) partials[blockIdx.x] = x;
+    x = block_fold<BLOCK>(x, s_waves, op);
+    if (tid == 0) partials[blockIdx.x] = gridDim.x == 1 ? op(init, x) : x;
 }
 
 // Folds `count` partials, then folds the result into the initial value: op(init, aggregate) (the type's
@@ -418,7 +425,7 @@ int reduce_sum(void* temp, size_t temp_bytes, const T* in, T* out, uint64_t n, v
     const uint64_t nvec = (n - head) / V;
 
     const uint64_t chunk = static_cast<uint64_t>(kReduceBlock) * kReduceUnroll;
-    uint64_t grid = ceil_div(nvec, chunk);
+    uint64_t grid = nvec <= kOneBlockVecs ? 1 : ceil_div(nvec, chunk);
     const uint64_t max_grid = static_cast<uint64_t>(device_cu_count()) * 8;
     if (grid > max_grid) grid = max_grid;
     if (grid < 1) grid = 1;
@@ -428,13 +435,16 @@ int reduce_sum(void* temp, size_t temp_bytes, const T* in, T* out, uint64_t n, v
 
     if (grid == 1) {
         LaunchScope scope("reduce_sum_partials", stream);
-        reduce_sum_partials_kernel<T><<<1, kReduceBlock, 0, stream>>>(in, n, static_cast<uint32_t>(head), nvec, out);
+        if (nvec <= chunk)
+            reduce_sum_partials_kernel<T, kReduceBlock><<<1, kReduceBlock, 0, stream>>>(in, n, static_cast<uint32_t>(head), nvec, out);
+        else
+            reduce_sum_partials_kernel<T, kOneBlock><<<1, kOneBlock, 0, stream>>>(in, n, static_cast<uint32_t>(head), nvec, out);
         return check_hip(hipGetLastError(), "reduce_sum_partials launch");
     }
     T* partials = static_cast<T*>(temp);
     {
         LaunchScope scope("reduce_sum_partials", stream);
-        reduce_sum_partials_kernel<T><<<static_cast<unsigned>(grid), kReduceBlock, 0, stream>>>(
+        reduce_sum_partials_kernel<T, kReduceBlock><<<static_cast<unsigned>(grid), kReduceBlock, 0, stream>>>(
             in, n, static_cast<uint32_t>(head), nvec, partials);
         int st = check_hip(hipGetLastError(), "reduce_sum_partials launch");
         if (st != kOk) return st;
@@ -446,19 +456,20 @@ int reduce_sum(void* temp, size_t temp_bytes, const T* in, T* out, uint64_t n, v
 
 // Grid of the persistent pass over n items at `in` (shared by every operator): the number of
 // unaligned leading items, the 16-byte vectors after them, and the workgroups (at most 8 per CU, at
-// most the partial slots the temp storage holds, one when it holds fewer than two).
+// most the partial slots the temp storage holds, one when it holds fewer than two or the input has at most
+// one_block_vecs vectors).
 struct ReducePlan {
     uint64_t head, nvec, grid;
 };
 template <typename T>
-ReducePlan reduce_plan(const T* in, uint64_t n, uint64_t partial_slots) {
+ReducePlan reduce_plan(const T* in, uint64_t n, uint64_t partial_slots, uint64_t one_block_vecs = 0) {
     constexpr int V = 16 / sizeof(T);
     const uintptr_t addr = reinterpret_cast<uintptr_t>(in);
     uint64_t head = ((16 - (addr & 15)) & 15) / sizeof(T);
     if (head > n) head = n;
     const uint64_t nvec = (n - head) / V;
     const uint64_t chunk = static_cast<uint64_t>(kReduceBlock) * kReduceUnroll;
-    uint64_t grid = ceil_div(nvec, chunk);
+    uint64_t grid = nvec <= one_block_vecs ? 1 : ceil_div(nvec, chunk);
     const uint64_t max_grid = static_cast<uint64_t>(device_cu_count()) * 8;
     if (grid > max_grid) grid = max_grid;
     if (grid < 1) grid = 1;
@@ -483,22 +494,20 @@ int reduce_generic(const char* what, const char* scope_name, void* temp, size_t 
     if (!in) return set_error(kInvalidArgument, "%s: null input", what);
     if (reinterpret_cast<uintptr_t>(in) % sizeof(T) != 0)
         return set_error(kInvalidArgument, "%s: input not aligned to its element size", what);
-    const ReducePlan pl = reduce_plan(in, n, temp ? temp_bytes / sizeof(T) : 0);
+    const ReducePlan pl = reduce_plan(in, n, temp ? temp_bytes / sizeof(T) : 0, kOneBlockVecs);
     T* partials = static_cast<T*>(temp);
     LaunchScope scope(scope_name, stream);
     if (pl.grid == 1) {
-        // One workgroup folds everything into the first temp slot (into *out when there is no temp);
-        // the final kernel then folds that value into the initial value.
-        T* slot = temp && temp_bytes >= sizeof(T) ? partials : out;
-        reduce_ext_partials_kernel<T, Op, XF><<<1, kReduceBlock, 0, stream>>>(in, n, static_cast<uint32_t>(pl.head),
-                                                                              pl.nvec, slot, scale, shift);
-        int st = check_hip(hipGetLastError(), "reduce launch");
-        if (st != kOk) return st;
-        reduce_ext_final_kernel<T, Op><<<1, kFinalBlock, 0, stream>>>(slot, 1u, init, out);
-        return check_hip(hipGetLastError(), "reduce final launch");
+        if (pl.nvec <= static_cast<uint64_t>(kReduceBlock) * kReduceUnroll)
+            reduce_ext_partials_kernel<T, Op, XF, kReduceBlock><<<1, kReduceBlock, 0, stream>>>(
+                in, n, static_cast<uint32_t>(pl.head), pl.nvec, out, scale, shift, init);
+        else
+            reduce_ext_partials_kernel<T, Op, XF, kOneBlock><<<1, kOneBlock, 0, stream>>>(
+                in, n, static_cast<uint32_t>(pl.head), pl.nvec, out, scale, shift, init);
+        return check_hip(hipGetLastError(), "reduce launch");
     }
-    reduce_ext_partials_kernel<T, Op, XF><<<static_cast<unsigned>(pl.grid), kReduceBlock, 0, stream>>>(
-        in, n, static_cast<uint32_t>(pl.head), pl.nvec, partials, scale, shift);
+    reduce_ext_partials_kernel<T, Op, XF, kReduceBlock><<<static_cast<unsigned>(pl.grid), kReduceBlock, 0, stream>>>(
+        in, n, static_cast<uint32_t>(pl.head), pl.nvec, partials, scale, shift, init);
     int st = check_hip(hipGetLastError(), "reduce launch");
     if (st != kOk) return st;
     reduce_ext_final_kernel<T, Op><<<1, kFinalBlock, 0, stream>>>(partials, static_cast<uint32_t>(pl.grid), init, out);
