@@ -909,10 +909,14 @@ uint32_t* longest_word(hipStream_t stream) {
 // Radix order with at least kWaveMean items per segment on average: a wave or a workgroup per segment
 // (segsort_waves.hip), which is faster from there on (per call, here and there: 4 M u32 + u32 pairs of mean 300
 // 203.8 -> 139.6 us, of mean 100 179.9 -> 129.7; 2^26 u32 of mean 100 1,136 -> 922, but of mean 40 953 -> 1,060,
-// where the joint sort of a tile fills its lanes better).
+// where the joint sort of a tile fills its lanes better).  Many medium segments of bare four-byte keys stream as well
+// there (2^26 u32 of mean 1,500: 1,102 us there, 1,116 here; 2^25 u32 pairs 811 and 768, u64 keys 1,151 and 1,154).
 constexpr uint64_t kWaveMean = 64;
+constexpr uint64_t kMediumMean = 1024, kMediumItems = 1u << 24;
+template <typename K, bool PAIRS>
 bool wave_route(uint64_t n, uint64_t num_segments, bool value_order) {
-    return !value_order && num_segments <= n / kWaveMean;
+    if (value_order || num_segments > n / kWaveMean) return false;
+    return PAIRS || sizeof(K) == 8 || num_segments > n / kMediumMean || n < kMediumItems;
 }
 
 template <typename K, typename V, bool PAIRS, int KIND>
@@ -942,7 +946,7 @@ int segsort(K* keys_in, K* keys_out, K* keys_scratch, V* values_in, V* values_ou
     const uint64_t cap = static_cast<uint64_t>(device_cu_count()) * 8;
     const uint64_t tile_cap = cap * 4;
     const unsigned tile_grid = static_cast<unsigned>(tiles < tile_cap ? tiles : tile_cap);
-    if (wave_route(n, num_segments, o.value_order)) {
+    if (wave_route<K, PAIRS>(n, num_segments, o.value_order)) {
         const SegmentKeys kind = KIND == kKindFloat ? SegmentKeys::kFloat
                                  : KIND == kKindSigned ? SegmentKeys::kSigned : SegmentKeys::kUnsigned;
         st = segsort_waves<K, V, PAIRS>(keys_in, keys_out, values_in, values_out, begins, ends, num_segments, n, kind,
