@@ -206,8 +206,9 @@ __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 
     while (small != 0) {
         const uint32_t from = static_cast<uint32_t>(__builtin_ctzll(small));
         small &= small - 1;
-        const uint64_t at = __builtin_amdgcn_readlane(b, from);
-        const uint32_t l = __builtin_amdgcn_readlane(len, from);
+        // wave_read_lane keeps the unsigned type: the builtin's int would be sign-extended from 2^31 on.
+        const uint64_t at = wave_read_lane(b, static_cast<int>(from));
+        const uint32_t l = wave_read_lane(len, static_cast<int>(from));
         if (l <= 64) wave_sort<U, V, PAIRS, 1>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
         else if (l <= 128) wave_sort<U, V, PAIRS, 2>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
         else if (l <= 256) wave_sort<U, V, PAIRS, 4>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);

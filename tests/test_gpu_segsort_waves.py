@@ -71,3 +71,36 @@ def test_double_buffer_in_place(hip, orc, dev):
     assert sel == (0, 0)
     np.testing.assert_array_equal(to_host(k0, np.uint32, n), wk)
     np.testing.assert_array_equal(to_host(v0, np.uint32, n), wv)
+
+
+def test_segments_on_both_sides_of_2p31(hip, dev):
+    """Offsets that a signed 32-bit word does not hold: one segment for each number of items per lane, and medium ones."""
+    n = (1 << 31) + 20_000
+    lengths = [40, 100, 200, 300, 512, 900, 4096]
+    b, e, at = [], [], (1 << 31) - sum(lengths) - 100
+    for x in lengths + [333] + lengths:  # the one in the middle straddles 2^31
+        b.append(at)
+        e.append(at + x)
+        at += x + 11
+    assert b[len(lengths)] < 1 << 31 < e[len(lengths)] and e[-1] <= n
+    first, last = b[0], e[-1]
+    rng = np.random.default_rng(5)
+    some = rng.integers(0, 1 << 32, last - first, dtype=np.uint64).astype(np.uint32)
+    keys = torch.zeros(n, dtype=torch.int32, device=dev)
+    keys[first:last] = to_dev(some)
+    vals = torch.zeros(n, dtype=torch.int32, device=dev)
+    vals[first:last] = torch.arange(last - first, dtype=torch.int32, device=dev)
+    ko, vo = torch.full_like(keys, -1), torch.full_like(vals, -1)
+    hip.segmented_sort("u32", keys, ko, n, len(b), to_dev(np.array(b, np.uint32)), to_dev(np.array(e, np.uint32)),
+                       values_in=vals, values_out=vo)
+    wk, wv = np.full(last - first, 0xFFFFFFFF, np.uint32), np.full(last - first, -1, np.int32)
+    for x, y in zip(b, e):
+        order = np.argsort(some[x - first:y - first], kind="stable")
+        wk[x - first:y - first] = some[x - first:y - first][order]
+        wv[x - first:y - first] = order + (x - first)
+    np.testing.assert_array_equal(ko[first:last].cpu().numpy().view(np.uint32), wk)
+    np.testing.assert_array_equal(vo[first:last].cpu().numpy(), wv)
+    for out in (ko, vo):  # nothing else is written
+        assert bool((out[:first] == -1).all()) and bool((out[last:] == -1).all())
+    del keys, vals, ko, vo, out
+    torch.cuda.empty_cache()
