@@ -343,6 +343,8 @@ __device__ __forceinline__ void radix_sort_chunk(const K* keys_in, K* kdst, cons
 
 // Radix order sorts chunks of up to kSsRadixChunk items in LDS; value order merges 2,048-item chunks.
 constexpr uint32_t kSsRadixChunk = 2 * kSsChunk;  // 4096
+// A segment above kSwMedium that were no longer than a chunk would be sorted by neither route's kernels.
+static_assert(kSwMedium == kSsRadixChunk, "segsort_waves leaves exactly the segments that the chunk kernel sorts");
 
 // Items sorted in LDS per chunk, the width the global passes start from, and the longest medium segment.
 __device__ __forceinline__ uint32_t chunk_items(const SortOrder& o) {

@@ -23,7 +23,7 @@ namespace {
 constexpr int kSwBlock = 512;
 constexpr int kSwWaves = kSwBlock / kWave;
 constexpr uint32_t kSwSmall = 512;    // items that one wave sorts
-constexpr uint32_t kSwMedium = 4096;  // items that the workgroup sorts
+// The workgroup sorts up to kSwMedium (segsort_waves.hpp).
 constexpr uint32_t kSwPerWave = kSwMedium / kSwWaves;
 static_assert(kSwSmall <= kSwPerWave, "a wave's share of the workgroup's arrays holds a small segment");
 

@@ -1,13 +1,15 @@
-// segsort_waves (segsort_waves.hip): sorts every segment of up to 4,096 items in radix order.
+// segsort_waves (segsort_waves.hip): sorts every segment of up to kSwMedium items in radix order.
 #pragma once
 
 #include "common.hpp"
 
 namespace lcpp_hip {
 
+constexpr uint32_t kSwMedium = 4096;  // items of the longest segment sorted here; segsort.hip sorts longer ones in chunks
+
 enum class SegmentKeys { kUnsigned, kSigned, kFloat };
 
-// Stable; in place when the outputs are the inputs.  Longer segments are left alone, and the length of the
+// Stable; in place when the outputs are the inputs.  Segments above kSwMedium are left alone, and the length of the
 // longest one is posted to words[0] when `words` is set.
 template <typename U, typename V, bool PAIRS>
 int segsort_waves(const U* keys_in, U* keys_out, const V* values_in, V* values_out, const uint32_t* begins,
