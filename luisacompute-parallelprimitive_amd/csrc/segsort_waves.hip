@@ -8,6 +8,7 @@
 //   * A wave sorts up to 512 items with no barrier: digits are ranked by ballot matches against the wave's own
 //     256 counters, four of which each lane scans, and the items move through the wave's own LDS.  Items per
 //     lane follow the length (1, 2, 4 or 8), since a rank step costs the same whether its items are real.
+//   * Tiny segments (up to 16 items) take a 16-lane row each, four at a time.
 //   * Medium segments are collected by the workgroup's waves and sorted by all 512 threads, 2, 4 or 8 items per
 //     thread.
 //   * Digits that are the same in a whole segment are skipped.
@@ -22,8 +23,10 @@ namespace {
 
 constexpr int kSwBlock = 512;
 constexpr int kSwWaves = kSwBlock / kWave;
+constexpr uint32_t kSwTiny = 16;      // items that a 16-lane row sorts
 constexpr uint32_t kSwSmall = 512;    // items that one wave sorts
 // The workgroup sorts up to kSwMedium (segsort_waves.hpp).
+constexpr uint32_t kSwPerWaveMost = 8;  // segments
 constexpr uint32_t kSwPerWave = kSwMedium / kSwWaves;
 static_assert(kSwSmall <= kSwPerWave, "a wave's share of the workgroup's arrays holds a small segment");
 
@@ -159,7 +162,59 @@ __device__ __forceinline__ void block_sort_segment(const U* keys_in, U* keys_out
     }
 }
 
-// Workgroup g takes the segments [g * per_group, (g + 1) * per_group), each wave per_wave (<= 64) of them, whose
+// Number of items before lane i's `key` among the `len` items of its 16-lane row: every rotation of the row (S = 1 ..
+// 15) brings another lane's key, with that lane's index.
+template <typename U, int S = 1>
+__device__ __forceinline__ uint32_t row_place(U key, uint32_t i, uint32_t len) {
+    if constexpr (S == 16) {
+        return 0;
+    } else {
+        constexpr int kRowRor = 0x120 + S;
+        const U other = dpp_move<kRowRor>(key, key);
+        const uint32_t j = dpp_move<kRowRor>(i, i);
+        const bool first = j < len && (other < key || (other == key && j < i));
+        return (first ? 1u : 0u) + row_place<U, S + 1>(key, i, len);
+    }
+}
+
+// Stable sorts of the tiny segments that the lanes in `tiny` hold, four at a time, one in each 16-lane row: every item
+// counts the items before it, which is its place.  About 80 instructions for four segments, without LDS; a wave sort of
+// each costs as much as one of 64 items (2^26 u32 pairs, 15 % of them in segments of 10 and the rest in segments of
+// 4,096, in random order: 1,184 -> 679 us per call).
+template <typename U, typename V, bool PAIRS>
+__device__ __forceinline__ void row_sorts(const U* keys_in, U* keys_out, const V* values_in, V* values_out, uint32_t b,
+                                          uint32_t len, uint64_t tiny, const SegmentBits<U>& sort_bits) {
+    const uint32_t lane = lane_id();
+    const uint32_t i = lane % 16;
+    while (tiny != 0) {
+        uint32_t begin = 0, l = 0;
+#pragma unroll
+        for (uint32_t row = 0; row < 4; ++row) {
+            if (tiny == 0) break;
+            const int from = __builtin_ctzll(tiny);
+            tiny &= tiny - 1;
+            const uint32_t rb = wave_read_lane(b, from), rl = wave_read_lane(len, from);
+            if (lane / 16 == row) {
+                begin = rb;
+                l = rl;
+            }
+        }
+        const uint64_t at = begin;
+        U k = 0;
+        V v = 0;
+        if (i < l) {
+            k = keys_in[at + i];
+            if constexpr (PAIRS) v = values_in[at + i];
+        }
+        const uint32_t place = row_place(sort_bits(k), i, l);
+        if (i < l) {
+            keys_out[at + place] = k;
+            if constexpr (PAIRS) values_out[at + place] = v;
+        }
+    }
+}
+
+// Workgroup g takes the segments [g * per_group, (g + 1) * per_group), each wave per_wave (<= kSwPerWaveMost) of them, whose
 // bounds its lanes read together.  The longest segment above kSwMedium goes to words[0] (a load first:
 // atomics on one address serialise).
 // 40 KB of LDS for four-byte pairs: three workgroups per CU, 24 waves, at most 80 VGPRs.
@@ -172,7 +227,7 @@ __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 
     static_assert(sizeof(U) * kSwSmall + (PAIRS ? sizeof(V) * kSwSmall : 0) + 1024 <= sizeof(typename Sorter::Shared) / kSwWaves,
                   "the waves' arrays fit the workgroup's");
     __shared__ __attribute__((aligned(16))) unsigned char s_lds[sizeof(typename Sorter::Shared)];
-    __shared__ uint16_t s_medium[kSwWaves * kWave];  // segments of the group, by number
+    __shared__ uint16_t s_medium[kSwWaves * kSwPerWaveMost];  // segments of the group, by number
     __shared__ uint32_t s_mediums, s_long;
     const uint32_t lane = lane_id();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -202,7 +257,9 @@ __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 
         keys_out[b] = keys_in[b];
         if constexpr (PAIRS) values_out[b] = values_in[b];
     }
-    uint64_t small = wave_ballot(len > 1 && len <= kSwSmall);
+    row_sorts<U, V, PAIRS>(keys_in, keys_out, values_in, values_out, b, len, wave_ballot(len > 1 && len <= kSwTiny),
+                           sort_bits);
+    uint64_t small = wave_ballot(len > kSwTiny && len <= kSwSmall);
     while (small != 0) {
         const uint32_t from = static_cast<uint32_t>(__builtin_ctzll(small));
         small &= small - 1;
@@ -245,9 +302,11 @@ int segsort_waves(const U* keys_in, U* keys_out, const V* values_in, V* values_o
     // Fewer than eight segments per workgroup while the workgroups do not fill the chip (three per CU): most of them
     // may be medium, and those of a workgroup are sorted one after the other (33 segments of mean 1,500: 105.8 us per
     // call with eight, 58.5 with one).  More than one per wave from four rounds of workgroups on, so that short
-    // segments cost a part of a workgroup's start.
+    // segments cost a part of a workgroup's start; at most eight, since where the long ones stand together their
+    // workgroups run alone at the end (2^26 u32 pairs, 13,926 segments of 4,096 items before 1,006,632 of 10: 4,602 us
+    // per call with 42 per wave, 1,419 with eight).
     const uint64_t resident = static_cast<uint64_t>(device_cu_count()) * 3;
-    const uint64_t per_wave = std::clamp<uint64_t>(num_segments / (resident * kSwWaves * 4), 1, kWave);
+    const uint64_t per_wave = std::clamp<uint64_t>(num_segments / (resident * kSwWaves * 4), 1, kSwPerWaveMost);
     const uint64_t per_group =
         per_wave > 1 ? per_wave * kSwWaves : std::clamp<uint64_t>(num_segments / resident, 1, kSwWaves);
     const uint64_t groups = ceil_div(num_segments, per_group);

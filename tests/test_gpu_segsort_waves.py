@@ -46,6 +46,22 @@ def test_lengths_at_the_edges(hip, orc, dev, ks, vb, desc):
         check(orc, keys, b, e, gk, gv, values=vals, **kw)
 
 
+@pytest.mark.parametrize("ks,vb", [("u32", 0), ("f32", 4), ("u32", 8), ("i64", 0), ("u64", 4), ("f64", 8)])
+@pytest.mark.parametrize("desc", [False, True])
+def test_tiny_segments(hip, orc, dev, ks, vb, desc):
+    """Segments of 1 to 17 items, a 16-lane row each up to 16, beside longer ones that keep the mean at 64 or more."""
+    rng = np.random.default_rng(vb + desc)
+    b, e, n = layout(rng, np.concatenate([np.arange(1, 18).repeat(40), np.full(700, 16), np.full(22, 4096), [300, 513, 1024]]))
+    assert len(b) <= n // 64
+    keys = words(rng, n, ks)
+    keys[::2] = keys[0]  # ties
+    vals = np.arange(n, dtype=np.uint32 if vb == 4 else np.uint64) if vb else None
+    for begin, end in [(0, 8 * keys.itemsize), (3, 17), (5, 5)]:
+        kw = dict(begin_bit=begin, end_bit=end, descending=desc)
+        gk, gv = g_sort(hip, keys, b, e, values=vals, **kw)
+        check(orc, keys, b, e, gk, gv, values=vals, **kw)
+
+
 def test_several_segments_per_wave(hip, orc, dev):
     rng = np.random.default_rng(3)
     b, e, n = layout(rng, np.concatenate([rng.integers(0, 150, 110_000), [513, 1500, 4096, 4097, 5000]]))
@@ -56,13 +72,15 @@ def test_several_segments_per_wave(hip, orc, dev):
     check(orc, keys, b, e, gk, gv, values=vals)
 
 
-def test_double_buffer_in_place(hip, orc, dev):
+@pytest.mark.parametrize("step,longest", [(1000, 1000), (70, 16)])
+def test_double_buffer_in_place(hip, orc, dev, step, longest):
     """ceil(log2 n) is even: the result goes where the input is."""
     rng = np.random.default_rng(4)
     n = 60_000
-    b = np.arange(0, n, 1000, dtype=np.uint32)
-    e = np.minimum(b + rng.integers(0, 1001, b.size), n).astype(np.uint32)
-    b, e = b[:60], e[:60]
+    b = np.arange(0, n, step, dtype=np.uint32)
+    e = np.minimum(b + rng.integers(0, longest + 1, b.size), n).astype(np.uint32)
+    if step == 1000:
+        b, e = b[:60], e[:60]
     keys, vals = words(rng, n, "u32"), np.arange(n, dtype=np.uint32)
     k0, v0 = to_dev(keys), to_dev(vals)
     k1, v1 = torch.zeros_like(k0), torch.zeros_like(v0)
