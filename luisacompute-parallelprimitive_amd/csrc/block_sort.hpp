@@ -72,21 +72,24 @@ struct BlockSort {
         const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
         const uint32_t first = wave * kWave * ITEMS + lane;
         const U vary = varying_bits(k, valid, sort_bits, s);
+        const bool idle = wave * kWave * ITEMS >= valid;  // no real item: the wave's counters stay zero
         uint32_t* const cnt = s.count[wave];
         for (uint32_t shift = 0; shift < bits; shift += 8) {
             if ((static_cast<uint32_t>(vary >> shift) & 0xFFu) == 0) continue;  // the same in every item
 #pragma unroll
             for (uint32_t i = 0; i < kBins / kWave; ++i) cnt[i * kWave + lane] = 0;
             uint32_t rank[ITEMS];  // digit << 16 | rank among the wave's items of that digit
+            if (!idle) {
 #pragma unroll
-            for (int j = 0; j < ITEMS; ++j) {
-                uint32_t d = static_cast<uint32_t>(sort_bits(k[j]) >> shift) & 0xFFu;
-                if (first + j * kWave >= valid) d = 0xFFu;
-                const uint64_t peers = match_digit(d);
-                const uint32_t below = popc_lanes_below(peers);
-                const uint32_t base = cnt[d];
-                rank[j] = (d << 16) | (base + below);
-                if ((peers >> lane) == 1ull) cnt[d] = base + below + 1;
+                for (int j = 0; j < ITEMS; ++j) {
+                    uint32_t d = static_cast<uint32_t>(sort_bits(k[j]) >> shift) & 0xFFu;
+                    if (first + j * kWave >= valid) d = 0xFFu;
+                    const uint64_t peers = match_digit(d);
+                    const uint32_t below = popc_lanes_below(peers);
+                    const uint32_t base = cnt[d];
+                    rank[j] = (d << 16) | (base + below);
+                    if ((peers >> lane) == 1ull) cnt[d] = base + below + 1;
+                }
             }
             __syncthreads();
             uint32_t before[kWaves];  // the digit's items in the waves before each wave
@@ -109,17 +112,21 @@ struct BlockSort {
                 for (int w = 0; w < kWaves; ++w) s.count[w][tid] = start + before[w];
             }
             __syncthreads();
+            if (!idle) {
 #pragma unroll
-            for (int j = 0; j < ITEMS; ++j) {
-                const uint32_t pos = cnt[rank[j] >> 16] + (rank[j] & 0xFFFFu);
-                s.key[pos] = k[j];
-                if constexpr (PAIRS) s.value[pos] = v[j];
+                for (int j = 0; j < ITEMS; ++j) {
+                    const uint32_t pos = cnt[rank[j] >> 16] + (rank[j] & 0xFFFFu);
+                    s.key[pos] = k[j];
+                    if constexpr (PAIRS) s.value[pos] = v[j];
+                }
             }
             __syncthreads();
+            if (!idle) {
 #pragma unroll
-            for (int j = 0; j < ITEMS; ++j) {
-                k[j] = s.key[first + j * kWave];
-                if constexpr (PAIRS) v[j] = s.value[first + j * kWave];
+                for (int j = 0; j < ITEMS; ++j) {
+                    k[j] = s.key[first + j * kWave];
+                    if constexpr (PAIRS) v[j] = s.value[first + j * kWave];
+                }
             }
         }
     }

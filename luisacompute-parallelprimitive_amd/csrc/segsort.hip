@@ -911,14 +911,22 @@ uint32_t* longest_word(hipStream_t stream) {
 // Radix order with at least kWaveMean items per segment on average: a wave or a workgroup per segment
 // (segsort_waves.hip), which is faster from there on (per call, here and there: 4 M u32 + u32 pairs of mean 300
 // 203.8 -> 139.6 us, of mean 100 179.9 -> 129.7; 2^26 u32 of mean 100 1,136 -> 922, but of mean 40 953 -> 1,060,
-// where the joint sort of a tile fills its lanes better).  Many medium segments of bare four-byte keys stream as well
-// there (2^26 u32 of mean 1,500: 1,102 us there, 1,116 here; 2^25 u32 pairs 811 and 768, u64 keys 1,151 and 1,154).
+// where the joint sort of a tile fills its lanes better).
 constexpr uint64_t kWaveMean = 64;
-constexpr uint64_t kMediumMean = 1024, kMediumItems = 1u << 24;
-template <typename K, bool PAIRS>
 bool wave_route(uint64_t n, uint64_t num_segments, bool value_order) {
-    if (value_order || num_segments > n / kWaveMean) return false;
-    return PAIRS || sizeof(K) == 8 || num_segments > n / kMediumMean || n < kMediumItems;
+    return !value_order && num_segments <= n / kWaveMean;
+}
+
+// Items of up to 8 bytes in many segments of more than kSsSmall items on average: the block kernel's 256 threads of up
+// to 16 items sort the medium ones faster than the wave kernel's 512 of up to 8, once they fill the chip and the second
+// launch is paid for (equal lengths, block kernel and wave kernel: 2^26 u32 pairs of 4,096 items 442 us
+// per call and 527, of 1,024 595 and 696; 2^26 u32 keys of 700 585 and 883; 2^22 u32 pairs of 1,024 64.9 and 69.9, but 2^20
+// 41.7 and 34.8, and log-normal lengths of mean 1,500 2^22 168.9 and 154.4, 2^26 1,283 and 1,311).  Wider items are faster
+// in the wave kernel: 2^26 u64 + u32 pairs of 1,024 items 1,839 and 1,713, 2^22 143.5 and 137.8.
+constexpr uint64_t kApartItems = 1u << 22;
+template <typename K, typename V, bool PAIRS>
+bool medium_apart(uint64_t n, uint64_t num_segments) {
+    return kSwApart<K, V, PAIRS> && n >= kApartItems && num_segments < n / kSsSmall;
 }
 
 template <typename K, typename V, bool PAIRS, int KIND>
@@ -948,30 +956,35 @@ int segsort(K* keys_in, K* keys_out, K* keys_scratch, V* values_in, V* values_ou
     const uint64_t cap = static_cast<uint64_t>(device_cu_count()) * 8;
     const uint64_t tile_cap = cap * 4;
     const unsigned tile_grid = static_cast<unsigned>(tiles < tile_cap ? tiles : tile_cap);
-    if (wave_route<K, PAIRS>(n, num_segments, o.value_order)) {
+    const bool waves = wave_route(n, num_segments, o.value_order);
+    const bool apart = waves && medium_apart<K, V, PAIRS>(n, num_segments);
+    if (waves) {
         const SegmentKeys kind = KIND == kKindFloat ? SegmentKeys::kFloat
                                  : KIND == kKindSigned ? SegmentKeys::kSigned : SegmentKeys::kUnsigned;
         st = segsort_waves<K, V, PAIRS>(keys_in, keys_out, values_in, values_out, begins, ends, num_segments, n, kind,
-                                        begin_bit, end_bit, descending != 0, words, stream);
+                                        begin_bit, end_bit, descending != 0, words, !apart, stream);
         if (st != kOk) return st;
-    } else {
+    }
+    if (!waves || apart) {
         // About one workgroup per 4,096 items (groups of segment offsets: with tiny and small segments each
         // workgroup reads many), but at least 8 per CU where the input allows, and never more than n / kSsSmall
         // (the most segments that can be medium).  Measured on 2^26 u32 keys against one per 512 items:
         // 16-item segments 0.80 -> 0.43 ms, 8-item pairs 0.95 -> 0.56, 1,024-item keys 0.474 -> 0.440.
+        // Up to 32 mostly medium segments per CU take a workgroup each (2^22 u32 pairs, log-normal lengths of mean 1,500:
+        // 167.9 us per call, 175.3 with two).
         const uint64_t most = n / kSsSmall > 0 ? n / kSsSmall : 1;
         const uint64_t fill = cap < most ? cap : most;
         const uint64_t target = n / (8 * kSsSmall) > fill ? n / (8 * kSsSmall) : fill;
-        const uint64_t per_group = ceil_div(num_segments, target);
+        const uint64_t per_group = apart && num_segments <= cap * 4 ? 1 : ceil_div(num_segments, target);
         const unsigned groups = static_cast<unsigned>(ceil_div(num_segments, per_group));
-        {
-            LaunchScope scope("segsort_block", stream);
-            segsort_block_kernel<K, V, PAIRS, KIND><<<groups, kSsBlock, 0, stream>>>(
-                keys_in, keys_out, values_in, values_out, begins, ends, static_cast<uint32_t>(num_segments),
-                static_cast<uint32_t>(per_group), n, o, words);
-            st = check_hip(hipGetLastError(), "segsort block launch");
-            if (st != kOk) return st;
-        }
+        LaunchScope scope("segsort_block", stream);
+        segsort_block_kernel<K, V, PAIRS, KIND><<<groups, kSsBlock, 0, stream>>>(
+            keys_in, keys_out, values_in, values_out, begins, ends, static_cast<uint32_t>(num_segments),
+            static_cast<uint32_t>(per_group), n, o, words);
+        st = check_hip(hipGetLastError(), "segsort block launch");
+        if (st != kOk) return st;
+    }
+    if (!waves) {
         // Tile and chunk kernels: grid-stride over 2,048-item tiles with enough workgroups to hide each
         // tile's segment searches; with no small (long) segment they exit after one word read.
         LaunchScope scope("segsort_tile", stream);

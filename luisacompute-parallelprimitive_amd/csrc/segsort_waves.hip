@@ -17,6 +17,7 @@
 #include "segsort_waves.hpp"
 
 #include <algorithm>
+#include <bit>
 
 namespace lcpp_hip {
 namespace {
@@ -214,29 +215,34 @@ __device__ __forceinline__ void row_sorts(const U* keys_in, U* keys_out, const V
     }
 }
 
-// Workgroup g takes the segments [g * per_group, (g + 1) * per_group), each wave per_wave (<= kSwPerWaveMost) of them, whose
-// bounds its lanes read together.  The longest segment above kSwMedium goes to words[0] (a load first:
+// Workgroup g takes the segments [g * per_group, (g + 1) * per_group), each wave per_wave (<= kSwPerWaveMost) of
+// them, whose bounds its lanes read together.  The longest segment above kSwMedium goes to words[0] (a load first:
 // atomics on one address serialise).
-// 40 KB of LDS for four-byte pairs: three workgroups per CU, 24 waves, at most 80 VGPRs.
-template <typename U, typename V, bool PAIRS>
+// 40 KB of LDS for four-byte pairs: three workgroups per CU, 24 waves, at most 80 VGPRs, for which the builds of u32 +
+// u32 pairs and u64 keys spill two and four (with 82 and none, two workgroups run: 2^26 u32 pairs in segments of 64
+// 658 -> 788 us per call).
+// MEDIUM: with the medium segments; without, the caller has them, the tiny ones and `words` done elsewhere.
+template <typename U, typename V, bool PAIRS, bool MEDIUM>
 __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 ? 6 : 4) void segsort_waves_kernel(
     const U* keys_in, U* keys_out, const V* values_in, V* values_out, const uint32_t* __restrict__ begins,
     const uint32_t* __restrict__ ends, uint32_t num_segments, uint32_t per_group, uint32_t per_wave, uint64_t n, uint32_t bits,
     SegmentBits<U> sort_bits, uint32_t* words) {
     using Sorter = BlockSort<U, V, PAIRS, kSwBlock, static_cast<int>(kSwMedium / kSwBlock)>;
-    static_assert(sizeof(U) * kSwSmall + (PAIRS ? sizeof(V) * kSwSmall : 0) + 1024 <= sizeof(typename Sorter::Shared) / kSwWaves,
-                  "the waves' arrays fit the workgroup's");
-    __shared__ __attribute__((aligned(16))) unsigned char s_lds[sizeof(typename Sorter::Shared)];
+    constexpr uint32_t kWaveBytes = 1024 + kSwSmall * (sizeof(U) + (PAIRS ? sizeof(V) : 0));
+    constexpr uint32_t kLdsBytes = MEDIUM ? sizeof(typename Sorter::Shared) : kSwWaves * kWaveBytes;
+    __shared__ __attribute__((aligned(16))) unsigned char s_lds[kLdsBytes];
+    static_assert(kWaveBytes <= sizeof(typename Sorter::Shared) / kSwWaves, "the waves' arrays fit the workgroup's");
     __shared__ uint16_t s_medium[kSwWaves * kSwPerWaveMost];  // segments of the group, by number
     __shared__ uint32_t s_mediums, s_long;
     const uint32_t lane = lane_id();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    if (threadIdx.x == 0) {
-        s_mediums = 0;
-        s_long = 0;
+    if constexpr (MEDIUM) {
+        if (threadIdx.x == 0) {
+            s_mediums = 0;
+            s_long = 0;
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    constexpr uint32_t kWaveBytes = 1024 + kSwSmall * (sizeof(U) + (PAIRS ? sizeof(V) : 0));
     unsigned char* const mine = s_lds + wave * kWaveBytes;
     const WaveLds<U, V, PAIRS> s{reinterpret_cast<U*>(mine + 1024), reinterpret_cast<V*>(mine + 1024 + kSwSmall * sizeof(U)),
                                  reinterpret_cast<uint32_t*>(mine)};
@@ -249,16 +255,23 @@ __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 
         const uint32_t e = ends[x];
         len = b < e && e <= n ? e - b : 0u;
     }
-    if (len > kSwMedium) {
-        atomicMax(&s_long, len);
-    } else if (len > kSwSmall) {
-        s_medium[atomicAdd(&s_mediums, 1u)] = static_cast<uint16_t>(member);
-    } else if (len == 1) {
-        keys_out[b] = keys_in[b];
-        if constexpr (PAIRS) values_out[b] = values_in[b];
+    if constexpr (MEDIUM) {
+        if (len > kSwMedium) {
+            atomicMax(&s_long, len);
+        } else if (len > kSwSmall) {
+            s_medium[atomicAdd(&s_mediums, 1u)] = static_cast<uint16_t>(member);
+        } else if (len == 1) {
+            keys_out[b] = keys_in[b];
+            if constexpr (PAIRS) values_out[b] = values_in[b];
+        }
     }
-    row_sorts<U, V, PAIRS>(keys_in, keys_out, values_in, values_out, b, len, wave_ballot(len > 1 && len <= kSwTiny),
-                           sort_bits);
+    // Where the tiny segments are sorted decides how the compiler lays out the sorts beside them: first costs
+    // 512-item segments of u32 + u64 pairs 9 % (2^26 items: 527 -> 575 us), last 4,096-item ones of u64 + u64 pairs
+    // 13 % (1,449 -> 1,640).
+    constexpr bool kTinyFirst = MEDIUM && sizeof(U) == 8;
+    if constexpr (kTinyFirst)
+        row_sorts<U, V, PAIRS>(keys_in, keys_out, values_in, values_out, b, len, wave_ballot(len > 1 && len <= kSwTiny),
+                               sort_bits);
     uint64_t small = wave_ballot(len > kSwTiny && len <= kSwSmall);
     while (small != 0) {
         const uint32_t from = static_cast<uint32_t>(__builtin_ctzll(small));
@@ -271,6 +284,10 @@ __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 
         else if (l <= 256) wave_sort<U, V, PAIRS, 4>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
         else wave_sort<U, V, PAIRS, 8>(keys_in, keys_out, values_in, values_out, at, l, bits, sort_bits, s);
     }
+    if constexpr (!MEDIUM) return;
+    if constexpr (!kTinyFirst)
+        row_sorts<U, V, PAIRS>(keys_in, keys_out, values_in, values_out, b, len, wave_ballot(len > 1 && len <= kSwTiny),
+                               sort_bits);
     __syncthreads();  // the list is complete, and the waves are done with their LDS
     const uint32_t mediums = s_mediums;
     for (uint32_t i = 0; i < mediums; ++i) {
@@ -291,7 +308,7 @@ __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 
 template <typename U, typename V, bool PAIRS>
 int segsort_waves(const U* keys_in, U* keys_out, const V* values_in, V* values_out, const uint32_t* begins,
                   const uint32_t* ends, uint64_t num_segments, uint64_t n, SegmentKeys kind, uint32_t begin_bit,
-                  uint32_t end_bit, bool descending, uint32_t* words, hipStream_t stream) {
+                  uint32_t end_bit, bool descending, uint32_t* words, bool medium, hipStream_t stream) {
     const uint32_t bits = end_bit - begin_bit;
     SegmentBits<U> sort_bits;
     sort_bits.float_mask = kind == SegmentKeys::kFloat ? static_cast<U>(~U(0)) : U(0);
@@ -299,27 +316,39 @@ int segsort_waves(const U* keys_in, U* keys_out, const V* values_in, V* values_o
     sort_bits.desc_mask = descending ? static_cast<U>(~U(0)) : U(0);
     sort_bits.bit_mask = bits == 0 ? U(0) : static_cast<U>(static_cast<U>(~U(0)) >> (sizeof(U) * 8 - bits));
     sort_bits.begin = bits == 0 ? 0u : begin_bit;
-    // Fewer than eight segments per workgroup while the workgroups do not fill the chip (three per CU): most of them
-    // may be medium, and those of a workgroup are sorted one after the other (33 segments of mean 1,500: 105.8 us per
-    // call with eight, 58.5 with one).  More than one per wave from four rounds of workgroups on, so that short
-    // segments cost a part of a workgroup's start; at most eight, since where the long ones stand together their
-    // workgroups run alone at the end (2^26 u32 pairs, 13,926 segments of 4,096 items before 1,006,632 of 10: 4,602 us
-    // per call with 42 per wave, 1,419 with eight).
+    // Workgroups that the chip holds together (three per CU).  Segments of more than kSwSmall items on average, of
+    // which a workgroup sorts one after the other: one per workgroup up to four rounds of workgroups, then two, four
+    // and eight (powers of two: 2^22 u32 + u64 pairs in segments of 1,024 take 90.5 us in groups of three, 84 in
+    // groups of two or four; 33 segments of mean 1,500, u32 pairs, took 105.8 us per call with eight and 58.5 with
+    // one; 4,194,304 u64 + u32 pairs in segments of 700 200.5 us with seven and 180.7 with one).  Shorter ones: one
+    // per workgroup while the workgroups do not fill the chip, then up to one per wave, and from four rounds of
+    // workgroups on more, so that they cost a part of a workgroup's start; at most eight per wave, since where the
+    // long ones stand together their workgroups run alone at the end (2^26 u32 pairs, 13,926 segments of 4,096 items
+    // before 1,006,632 of 10: 4,602 us per call with 42 per wave, 1,351 with eight).
     const uint64_t resident = static_cast<uint64_t>(device_cu_count()) * 3;
-    const uint64_t per_wave = std::clamp<uint64_t>(num_segments / (resident * kSwWaves * 4), 1, kSwPerWaveMost);
+    const bool mostly_medium = n / num_segments > kSwSmall;
+    const uint64_t per_wave =
+        mostly_medium ? 1 : std::clamp<uint64_t>(num_segments / (resident * kSwWaves * 4), 1, kSwPerWaveMost);
     const uint64_t per_group =
-        per_wave > 1 ? per_wave * kSwWaves : std::clamp<uint64_t>(num_segments / resident, 1, kSwWaves);
+        per_wave > 1 || !medium ? per_wave * kSwWaves
+        : mostly_medium        ? std::bit_floor(std::clamp<uint64_t>(num_segments / (resident * 4), 1, kSwWaves))
+                               : std::clamp<uint64_t>(num_segments / resident, 1, kSwWaves);
     const uint64_t groups = ceil_div(num_segments, per_group);
     LaunchScope scope("segsort_waves", stream);
-    segsort_waves_kernel<U, V, PAIRS><<<static_cast<unsigned>(groups), kSwBlock, 0, stream>>>(
-        keys_in, keys_out, values_in, values_out, begins, ends, static_cast<uint32_t>(num_segments),
-        static_cast<uint32_t>(per_group), static_cast<uint32_t>(per_wave), n, bits, sort_bits, words);
+    const auto launch = [&](auto kernel) {
+        kernel<<<static_cast<unsigned>(groups), kSwBlock, 0, stream>>>(
+            keys_in, keys_out, values_in, values_out, begins, ends, static_cast<uint32_t>(num_segments),
+            static_cast<uint32_t>(per_group), static_cast<uint32_t>(per_wave), n, bits, sort_bits, words);
+    };
+    if (medium) launch(segsort_waves_kernel<U, V, PAIRS, true>);
+    else if constexpr (kSwApart<U, V, PAIRS>) launch(segsort_waves_kernel<U, V, PAIRS, false>);
     return check_hip(hipGetLastError(), "segsort waves launch");
 }
 
 #define LCPP_HIP_SEGSORT_WAVES(U, V, P)                                                                            \
     template int segsort_waves<U, V, P>(const U*, U*, const V*, V*, const uint32_t*, const uint32_t*, uint64_t,    \
-                                        uint64_t, SegmentKeys, uint32_t, uint32_t, bool, uint32_t*, hipStream_t);
+                                        uint64_t, SegmentKeys, uint32_t, uint32_t, bool, uint32_t*, bool,              \
+                                        hipStream_t);
 LCPP_HIP_SEGSORT_WAVES(uint32_t, uint32_t, false)
 LCPP_HIP_SEGSORT_WAVES(uint32_t, uint32_t, true)
 LCPP_HIP_SEGSORT_WAVES(uint32_t, uint64_t, true)

@@ -72,6 +72,27 @@ def test_several_segments_per_wave(hip, orc, dev):
     check(orc, keys, b, e, gk, gv, values=vals)
 
 
+@pytest.mark.parametrize("ks,vb", [("u32", 0), ("f32", 4), ("i32", 4), ("i64", 0)])
+@pytest.mark.parametrize("desc", [False, True])
+def test_medium_segments_apart(hip, orc, dev, ks, vb, desc):
+    """Items of up to 8 bytes, 2^22 of them or more, more than 512 per segment: the block kernel sorts the tiny and the medium
+    segments, the wave kernel those between."""
+    rng = np.random.default_rng(vb + desc)
+    b, e, n = layout(rng, np.concatenate([EDGES * 3, np.arange(1, 18), rng.integers(513, 4097, 1000)]).astype(np.int64))
+    n = max(n, 1 << 22)
+    assert len(b) < n // 512  # on average
+    keys = words(rng, n, ks)
+    vals = np.arange(n, dtype=np.uint32) if vb else None
+    for begin, end in [(0, 8 * keys.itemsize), (3, 17), (5, 5)]:
+        kw = dict(begin_bit=begin, end_bit=end, descending=desc)
+        hip.profile_reset()
+        hip.profile_enable(True)
+        gk, gv = g_sort(hip, keys, b, e, values=vals, **kw)
+        hip.profile_enable(False)
+        assert [hip.profile_query(f"segsort_{x}")[1] for x in ("block", "waves", "tile")] == [1, 1, 0]
+        check(orc, keys, b, e, gk, gv, values=vals, **kw)
+
+
 @pytest.mark.parametrize("step,longest", [(1000, 1000), (70, 16)])
 def test_double_buffer_in_place(hip, orc, dev, step, longest):
     """ceil(log2 n) is even: the result goes where the input is."""
