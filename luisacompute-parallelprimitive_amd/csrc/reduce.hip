@@ -34,22 +34,31 @@ template <typename T>
 using Vec16 = T __attribute__((ext_vector_type(16 / sizeof(T))));
 
 // Inputs of up to one round of a 1,024-thread workgroup (64 KB) are folded by that workgroup alone: the second
-// launch costs more than the CUs it leaves idle (5,003 f32 9.8 -> 7.9 us per call, 16,384
-// 10.3 -> 7.8).
+// launch costs more than the CUs it leaves idle (5,003 f32 9.8 -> 7.9 us per call, 16,384 10.3 -> 7.8).  Its four
+// teams of kReduceBlock threads take the items that four workgroups would, and their folds meet pairwise, as the final
+// kernel's first lanes do it: the result is that of the two launches, bit for bit.  (All 1,024 threads side by side,
+// with the 16 waves' sums added one after the other, raised the mean error of uniform f32 sums 1.2 to 1.5 times.)
 constexpr int kOneBlock = 1024;
+constexpr int kTeamWaves = kReduceBlock / kWave;
 constexpr uint64_t kOneBlockVecs = static_cast<uint64_t>(kOneBlock) * kReduceUnroll;
 
 template <int BLOCK, typename T>
 __device__ __forceinline__ T block_sum(T x, T* s_waves) {
     constexpr int W = BLOCK / kWave;
+    static_assert(W == kTeamWaves || W == 4 * kTeamWaves, "one team or four");
     x = wave_reduce(x, SumOp{});
     const int wave = threadIdx.x / kWave;
     if (lane_id() == 0) s_waves[wave] = x;
     __syncthreads();
-    T total = s_waves[0];
+    T total[W / kTeamWaves];
 #pragma unroll
-    for (int w = 1; w < W; ++w) total += s_waves[w];
-    return total;
+    for (int g = 0; g < W / kTeamWaves; ++g) {
+        total[g] = s_waves[g * kTeamWaves];
+#pragma unroll
+        for (int w = 1; w < kTeamWaves; ++w) total[g] += s_waves[g * kTeamWaves + w];
+    }
+    if constexpr (W == kTeamWaves) return total[0];
+    else return (total[0] + total[1]) + (total[2] + total[3]);
 }
 
 // Folds in[0..n) into partials[blockIdx.x].  `head` leading elements precede the first 16-byte
@@ -68,13 +77,15 @@ __global__ __launch_bounds__(BLOCK) void reduce_sum_partials_kernel(const T* __r
 #pragma unroll
     for (int u = 0; u < kReduceUnroll; ++u) acc[u] = T(0);
 
-    const uint64_t chunk = static_cast<uint64_t>(BLOCK) * kReduceUnroll;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * chunk;
-    uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunk;
+    constexpr uint32_t kTeams = BLOCK / kReduceBlock;
+    const uint32_t team = tid / kReduceBlock, at = tid % kReduceBlock;
+    const uint64_t chunk = static_cast<uint64_t>(kReduceBlock) * kReduceUnroll;
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kTeams * chunk;
+    uint64_t base = (static_cast<uint64_t>(blockIdx.x) * kTeams + team) * chunk;
     for (; base + chunk <= nvec; base += stride) {
         Vec v[kReduceUnroll];
 #pragma unroll
-        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * BLOCK + tid]);
+        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * kReduceBlock + at]);
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
             T s = v[u][0];
@@ -86,7 +97,7 @@ __global__ __launch_bounds__(BLOCK) void reduce_sum_partials_kernel(const T* __r
     if (base < nvec) {  // last, partial chunk of this workgroup
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
-            const uint64_t idx = base + u * BLOCK + tid;
+            const uint64_t idx = base + u * kReduceBlock + at;
             if (idx < nvec) {
                 Vec v = vin[idx];
                 T s = v[0];
@@ -178,14 +189,20 @@ struct WrapSumOp {
 template <int BLOCK, typename T, typename Op>
 __device__ __forceinline__ T block_fold(T x, T* s_waves, Op op) {
     constexpr int W = BLOCK / kWave;
+    static_assert(W == kTeamWaves || W == 4 * kTeamWaves, "one team or four");
     x = wave_reduce(x, op);
     const int wave = threadIdx.x / kWave;
     if (lane_id() == 0) s_waves[wave] = x;
     __syncthreads();
-    T total = s_waves[0];
+    T total[W / kTeamWaves];
 #pragma unroll
-    for (int w = 1; w < W; ++w) total = op(total, s_waves[w]);
-    return total;
+    for (int g = 0; g < W / kTeamWaves; ++g) {
+        total[g] = s_waves[g * kTeamWaves];
+#pragma unroll
+        for (int w = 1; w < kTeamWaves; ++w) total[g] = op(total[g], s_waves[g * kTeamWaves + w]);
+    }
+    if constexpr (W == kTeamWaves) return total[0];
+    else return op(op(total[0], total[1]), op(total[2], total[3]));
 }
 
 // reduce_sum_partials_kernel with another operator (min / max, or the sum in the item's own type) and a
@@ -205,13 +222,15 @@ __global__ __launch_bounds__(BLOCK) void reduce_ext_partials_kernel(const T* __r
     T acc[kReduceUnroll];
 #pragma unroll
     for (int u = 0; u < kReduceUnroll; ++u) acc[u] = Op::template identity<T>();
-    const uint64_t chunk = static_cast<uint64_t>(BLOCK) * kReduceUnroll;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * chunk;
-    uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunk;
+    constexpr uint32_t kTeams = BLOCK / kReduceBlock;
+    const uint32_t team = tid / kReduceBlock, at = tid % kReduceBlock;
+    const uint64_t chunk = static_cast<uint64_t>(kReduceBlock) * kReduceUnroll;
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kTeams * chunk;
+    uint64_t base = (static_cast<uint64_t>(blockIdx.x) * kTeams + team) * chunk;
     for (; base + chunk <= nvec; base += stride) {
         Vec v[kReduceUnroll];
 #pragma unroll
-        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * BLOCK + tid]);
+        for (int u = 0; u < kReduceUnroll; ++u) v[u] = __builtin_nontemporal_load(&vin[base + u * kReduceBlock + at]);
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
 #pragma unroll
@@ -221,7 +240,7 @@ __global__ __launch_bounds__(BLOCK) void reduce_ext_partials_kernel(const T* __r
     if (base < nvec) {
 #pragma unroll
         for (int u = 0; u < kReduceUnroll; ++u) {
-            const uint64_t idx = base + u * BLOCK + tid;
+            const uint64_t idx = base + u * kReduceBlock + at;
             if (idx < nvec) {
                 const Vec v = vin[idx];
 #pragma unroll
