@@ -19,9 +19,9 @@
 // MI355X design
 //   * Tile = 256 threads x R rows x 4 consecutive items per thread and row (R = 12 for 4-byte keys and
 //     values in the scan, 15 in the reduce, 22 in the count mode: 12,288 / 15,360 / 22,528 items; fewer
-//     for 8-byte types, and 4 rows for smaller inputs), every row a contiguous 1,024 items read (and, for the scan, written) with
-//     16-byte vectors, all rows' loads in flight together; four workgroups per CU (three for the
-//     reduce).  The key before a thread-row is the previous
+//     for 8-byte types and for smaller inputs), every row a contiguous 1,024 items read (and, for the
+//     scan, written) with 16-byte vectors, all rows' loads in flight together; four workgroups per CU
+//     (three for the reduce).  The key before a thread-row is the previous
 //     lane's last key (DPP wave shift) or, for lane 0, the last key of the previous wave or row (a
 //     small LDS table).
 //   * State of a span of items: (heads, sum since the last head).  States combine as
@@ -106,14 +106,26 @@ constexpr int kBkRows =
 template <typename K, typename V>
 constexpr uint32_t kBkStageItems = 32768u / static_cast<uint32_t>(sizeof(K) + sizeof(V));
 // Inputs of up to kBkSmallItems take tiles of 4 rows (4,096 items), enough of them to fill the chip.  Reduces and run
-// lengths, whose walk needs every earlier tile's count, read a whole wave of states per step there, since those
-// tiles run and publish together; a scan's walk mostly ends at the nearest head, and 8 states per step serve it up
-// to where its larger tiles stream as well.  Per call, full-size tiles -> 4 rows: ReduceByKey i32 / f32, runs of 20,
-// 1,000,003 items 15.3 -> 12.2 us, 4,000,037 19.3 -> 15.0, but 6,000,001 19.1 -> 20.9 (runs of 64; i64 / f64 2 M
-// 18.0 -> 16.9, 4 M 25.8 -> 30.0); encode u32, runs of 8, 1,000,003 18.9 -> 11.9, 4,000,037 21.4 -> 14.6, unique
-// 6,000,001 19.4 -> 18.5, encode 10,000,019 23.7 -> 29.1; ExclusiveSumByKey 1,000,003 15.7 -> 11.9, 4,000,037 18.4 ->
-// 12.7, 20,000,003 48.3 -> 44.9, 40,000,003 88.2 -> 82.8 (i64 / f64 6 M 39.7 -> 35.7).
+// lengths, whose walk needs every earlier tile's count, read a whole wave of states per step there, since those tiles
+// run and publish together.  A scan's walk ends at the nearest head: 8 states find it where runs are short, and a
+// walk that goes on reads kBkWindow per step.  (8 all the way: 1,000,003 items in one run 14.0 us per call, 4,000,037
+// 22.6; with 32 from the second step on 12.2 and 18.3; full-size tiles 14.6 and 17.9.)  Per call, full-size tiles -> 4
+// rows: ReduceByKey i32 / f32, runs of 20, 1,000,003 items 15.3 -> 12.2 us, 4,000,037 19.3 -> 15.0, but 6,000,001
+// 19.1 -> 20.9 (runs of 64; i64 / f64 2 M 18.0 -> 16.9, 4 M 25.8 -> 30.0); encode u32, runs of 8, 1,000,003 18.9 ->
+// 11.9, 4,000,037 21.4 -> 14.6, unique 6,000,001 19.4 -> 18.5, encode 10,000,019 23.7 -> 29.1; ExclusiveSumByKey
+// 1,000,003 15.7 -> 11.9, 4,000,037 18.4 -> 12.7.
+// Larger scans' long runs are walked over many tiles, so scans of more than 64 MB of keys and values of up to 12 bytes
+// take fewer, of kBkMidRows rows, which stream short runs nearly as fast (full-size tiles, 4 rows and 6, us per call of
+// i32 / u32: 10,000,019 items in runs of 20 32.6, 26.8 and 27.7, of 1,000,000 31.2, 32.0 and 32.8, in one 27.4, 34.4
+// and 32.8; 41,000,001 items 94.6, 86.6 and 87.3, 96.8, 109.2 and 101.2, 98.5, 116.1 and 105.5; 8 rows take 28.3 us for
+// the first and 102.1 for the last; i32 / f64, 20,000,003 items, 99.5, 87.8 and 90.3, 107.6, 106.1 and 98.6, 108.1,
+// 110.5 and 100.8).  16-byte items keep 4 rows, which are not behind (i64 / f64, 41,000,001 items 226.8 and 209.6, 254.1
+// and 241.2, 257.7 and 247.9).
 constexpr int kBkSmallRows = 4;
+template <typename K, typename V>
+constexpr int kBkMidRows = sizeof(K) + sizeof(V) <= 12 ? 6 : kBkSmallRows;
+template <typename K, typename V>
+constexpr uint64_t kBkMidItems = (64ull << 20) / (sizeof(K) + sizeof(V));
 template <typename K, typename V, int MODE>
 constexpr uint64_t kBkSmallItems = MODE == 0   ? 42'000'000
                                    : MODE == 1 ? (32ull << 20) / (sizeof(K) + sizeof(V))
@@ -522,7 +534,7 @@ __global__ __launch_bounds__(kBkBlock, kBkBlocksPerCu<MODE>) void by_key_kernel(
     const K* __restrict__ keys, const V* values_in, V* values_out, K* __restrict__ unique_out,
     V* __restrict__ aggregates_out, uint32_t* __restrict__ num_runs_out, uint64_t n, K mask,
     uint64_t* __restrict__ states, int inclusive, int use_init, V init, bool vec_k, bool vec_v, bool vec_o,
-    bool in_place, uint32_t spin_limit, uint32_t look_window) {
+    bool in_place, uint32_t spin_limit, uint32_t first_window, uint32_t next_window) {
     constexpr bool COUNTED = MODE != kModeScan;
     constexpr int W = kStateWords<V, COUNTED>;
     uint64_t* const claims = states + static_cast<uint64_t>(gridDim.x) * W;
@@ -707,6 +719,7 @@ __global__ __launch_bounds__(kBkBlock, kBkBlocksPerCu<MODE>) void by_key_kernel(
     Seg<V> prefix{0u, op_identity<Op, V>()};
     if (tile > 0) {
         int64_t top = static_cast<int64_t>(tile) - 1;  // newest predecessor not yet consumed
+        uint32_t look_window = first_window;            // states read per step
         Seg<V> acc{0u, op_identity<Op, V>()};           // states consumed so far (wave 0)
         uint32_t spins = 0;
         uint32_t row = 0;
@@ -761,6 +774,7 @@ __global__ __launch_bounds__(kBkBlock, kBkBlocksPerCu<MODE>) void by_key_kernel(
             if (action == kActDone) break;
             if (action == kActAdvance) {
                 top -= look_window;
+                if constexpr (MODE == kModeScan) look_window = next_window;
                 spins = 0;
                 continue;
             }
@@ -889,7 +903,7 @@ int by_key(void* temp, size_t temp_bytes, const K* keys, const V* values_in, V* 
     if (!temp || temp_bytes < need)
         return set_error(kTempTooSmall, "%s: temp storage too small (%zu < %zu bytes)", what, temp_bytes, need);
     if (reinterpret_cast<uintptr_t>(temp) % 8 != 0) return set_error(kInvalidArgument, "%s: temp not 8-byte aligned", what);
-    const auto launch = [&](auto rows, uint32_t window) {
+    const auto launch = [&](auto rows, uint32_t first_window, uint32_t next_window) {
         constexpr int R = decltype(rows)::value;
         constexpr uint32_t kTile = static_cast<uint32_t>(kBkBlock * kBkVec * R);
         uint64_t* states = static_cast<uint64_t*>(temp);
@@ -901,13 +915,22 @@ int by_key(void* temp, size_t temp_bytes, const K* keys, const V* values_in, V* 
         by_key_kernel<K, V, MODE, R, Op><<<tiles, kBkBlock, 0, stream>>>(
             keys, values_in, values_out, unique_out, aggregates_out, num_runs_out, n, static_cast<K>(key_mask), states,
             inclusive, use_init, init, aligned16(keys), aligned16(values_in), values_out != nullptr && aligned16(values_out),
-            values_out != nullptr && values_out == values_in, lookback_spin_limit(), window);
+            values_out != nullptr && values_out == values_in, lookback_spin_limit(), first_window, next_window);
         return check_hip(hipGetLastError(), MODE == kModeScan ? "scan_by_key launch" : "reduce_by_key launch");
     };
-    if (n <= kBkSmallItems<K, V, MODE> &&
-        temp_bytes >= state_bytes(n, kBkBlock * kBkVec * kBkSmallRows, sizeof(V), MODE != kModeScan))
-        return launch(std::integral_constant<int, kBkSmallRows>{}, MODE == kModeScan ? 8u : static_cast<uint32_t>(kWave));
-    return launch(std::integral_constant<int, kRows>{}, static_cast<uint32_t>(kBkWindow));
+    constexpr uint32_t kWindow = kBkWindow;
+    const auto fits = [&](int rows) {
+        return temp_bytes >= state_bytes(n, static_cast<uint32_t>(kBkBlock * kBkVec * rows), sizeof(V), MODE != kModeScan);
+    };
+    if constexpr (MODE == kModeScan) {
+        constexpr int kMid = kBkMidRows<K, V>;
+        if (kMid != kBkSmallRows && n > kBkMidItems<K, V> && n <= kBkSmallItems<K, V, MODE> && fits(kMid))
+            return launch(std::integral_constant<int, kMid>{}, 8u, kWindow);
+    }
+    if (n <= kBkSmallItems<K, V, MODE> && fits(kBkSmallRows))
+        return launch(std::integral_constant<int, kBkSmallRows>{}, MODE == kModeScan ? 8u : static_cast<uint32_t>(kWave),
+                      MODE == kModeScan ? kWindow : static_cast<uint32_t>(kWave));
+    return launch(std::integral_constant<int, kRows>{}, kWindow, kWindow);
 }
 
 }  // namespace

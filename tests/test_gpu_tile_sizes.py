@@ -97,3 +97,23 @@ def test_scan_by_key_where_the_tiles_change(hip, dev, n):
     hip.scan_by_key("i32", "i32", to_dev(key), to_dev(x), out, n)
     s = np.cumsum(x) - x
     np.testing.assert_array_equal(out.cpu().numpy(), (s - s[::1000][key]).astype(np.int32))
+
+
+@pytest.mark.parametrize("k,t,n", [(k, t, n) for k, t, b in [("i32", "u32", 8), ("i64", "i32", 12), ("u32", "i64", 12),
+                                                             ("u64", "u64", 16)]
+                                   for n in around((64 << 20) // b, 1400 * 6144)])
+def test_scan_by_key_mid_tiles(hip, dev, spin, k, t, n):
+    """Above 64 MB of keys and values the tiles have 6 rows (items of 8 and 12 bytes); runs within a tile, over more tiles
+    than one look-back step reads, and a single one, out of place and in place."""
+    np_t = np.dtype({"u": np.uint32, "i": np.int32}[t[0]] if t[1:] == "32" else {"u": np.uint64, "i": np.int64}[t[0]])
+    x = np.random.default_rng(n).integers(0, 50, n).astype(np_t)
+    s = np.cumsum(x, dtype=np_t)
+    for run in (1000, 700_001, n):
+        at = np.arange(n) // run
+        start = (s - x)[::run][at]
+        dk, dx = to_dev(at.astype(np.int64 if k[1:] == "64" else np.int32)), to_dev(x)
+        out = torch.zeros_like(dx)
+        hip.scan_by_key(k, t, dk, dx, out, n)
+        np.testing.assert_array_equal(out.cpu().numpy().view(np_t), s - x - start)
+        hip.scan_by_key(k, t, dk, dx, dx, n, inclusive=True)
+        np.testing.assert_array_equal(dx.cpu().numpy().view(np_t), s - start)
