@@ -755,7 +755,11 @@ constexpr int kSelRows = (FLAGS || sizeof(U) == 8) ? 12 : 16;
 // Select-if of u32, a third kept, per call with 16 rows and 8 states / 8 rows and 64 / 4 rows and 64:
 // 1,000,003 items 19.2 / 13.1 / 12.8 us, 4,000,037 22.6 / 15.5 / 13.7, 6,000,003 25.1 / 18.4 / 17.6, 10,000,019
 // 29.0 / 22.0 / 25.3, 40,000,003 73.8 / 63.5 / 78.6; partition of 64 M 113.8 / 122.4; 20 M u64 66.0 / 64.5 / 82.8.
-constexpr uint64_t kSel4Tiles = 1536, kSel8Tiles = 5120;
+// 8-byte items with flags, or all of them written, stream as well over the full-size tiles from 3,584 8-row tiles on
+// (12 rows / 8 rows: partition of 12,000,001 48.7 / 46.8, 14,000,001 59.5 / 59.7, 20,000,003 75.9 / 81.0; with byte
+// flags, half kept, 45.4 / 44.9, 50.3 / 50.1, 68.4 / 70.2; select-if of 20,000,003, a tenth kept 63.0 / 57.0, 0.95 kept
+// 74.3 / 79.0).
+constexpr uint64_t kSel4Tiles = 1536, kSel8Tiles = 5120, kSel8DenseTiles = 3584;
 template <typename U, int R>
 constexpr uint32_t kRowsTile = static_cast<uint32_t>(kRowsBlock) * R * kRowItems<U>;
 
@@ -1243,7 +1247,8 @@ int run_compact(const char* what, void* temp, size_t temp_bytes, const U* in, co
             };
             if (n <= static_cast<uint64_t>(kRowsTile<U, 4>) * kSel4Tiles && temp_bytes >= plan_temp(n, kRowsTile<U, 4>, 1, 0).total)
                 return launch(std::integral_constant<int, 4>{}, kWave);
-            if (n <= static_cast<uint64_t>(kRowsTile<U, 8>) * kSel8Tiles && temp_bytes >= plan_temp(n, kRowsTile<U, 8>, 1, 0).total)
+            const uint64_t tiles8 = sizeof(U) == 8 && (FLAGS || a.partition) ? kSel8DenseTiles : kSel8Tiles;
+            if (n <= static_cast<uint64_t>(kRowsTile<U, 8>) * tiles8 && temp_bytes >= plan_temp(n, kRowsTile<U, 8>, 1, 0).total)
                 return launch(std::integral_constant<int, 8>{}, kWave);
             return launch(std::integral_constant<int, kSelRows<U, FLAGS>>{}, kRowsWindow);
         }

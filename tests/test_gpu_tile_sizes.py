@@ -56,6 +56,47 @@ def test_select_everything(hip, dev, t, n):
     assert not out[n:].any()
 
 
+FLAGGED = [("u32", n) for n in around(4096, 1536 * 4096) + [5120 * 8192, 5120 * 8192 + 1]] + \
+          [("u64", n) for n in around(2048, 1536 * 2048, 3584 * 4096)]
+
+
+@pytest.mark.parametrize("t,n", FLAGGED)
+@pytest.mark.parametrize("fs", ["b8", "u32"])
+def test_flagged(hip, dev, spin, t, n, fs):
+    """Select and partition by flags, over tiles of 4, 8 and 12 rows."""
+    np_t = np.uint32 if t == "u32" else np.uint64
+    rng = np.random.default_rng(n)
+    x = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np_t)
+    keep = rng.random(n, dtype=np.float32) < 0.6
+    d, num = to_dev(x), torch.zeros(1, dtype=torch.int32, device=dev)
+    flags = to_dev(keep.astype(np.uint8 if fs == "b8" else np.uint32))
+    k = int(keep.sum())
+    for call in (hip.select_flagged, hip.partition_flagged):
+        out = torch.zeros_like(d)
+        call(t, fs, d, flags, out, num, n)
+        assert int(num.item()) == k
+        got = out.cpu().numpy().view(np_t)
+        np.testing.assert_array_equal(got[:k], x[keep])
+        np.testing.assert_array_equal(got[k:], x[~keep][::-1] if call is hip.partition_flagged else 0)
+
+
+@pytest.mark.parametrize("n", [5] + around(2048, 1536 * 2048, 3584 * 4096, 5120 * 4096))
+def test_select_and_partition_8_byte(hip, dev, spin, n):
+    """The 8-byte items' row counts (4, 8, 12) with a predicate that keeps a part."""
+    x = np.random.default_rng(n).integers(0, 1 << 63, n, dtype=np.uint64) << np.uint64(1)
+    bound = 0xA000000000000000
+    d, num = to_dev(x), torch.zeros(1, dtype=torch.int32, device=dev)
+    keep = x < np.uint64(bound)
+    k = int(keep.sum())
+    for call in (hip.select_if, hip.partition_if):
+        out = torch.zeros_like(d)
+        call("u64", d, out, num, n, hip.predicate("u64", (hip.PRED_LT, bound)))
+        assert int(num.item()) == k
+        got = out.cpu().numpy().view(np.uint64)
+        np.testing.assert_array_equal(got[:k], x[keep])
+        np.testing.assert_array_equal(got[k:], x[~keep][::-1] if call is hip.partition_if else 0)
+
+
 RUNS = [1, 3] + around(4096, 64 * 4096, (32 << 20) // 8, (24 << 20) // 4)
 
 
