@@ -141,7 +141,7 @@ template <typename U, typename V, bool PAIRS, int ITEMS>
 __device__ __forceinline__ void block_sort_segment(const U* keys_in, U* keys_out, const V* values_in, V* values_out,
                                                    uint64_t at, uint32_t len, uint32_t bits,
                                                    const SegmentBits<U>& sort_bits, unsigned char* lds) {
-    using Sorter = BlockSort<U, V, PAIRS, kSwBlock, ITEMS>;
+    using Sorter = BlockSort<U, V, PAIRS, kSwBlock, ITEMS, true>;
     const uint32_t first = threadIdx.x / kWave * kWave * ITEMS + lane_id();
     U k[ITEMS];
     V v[PAIRS ? ITEMS : 1];
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kSwBlock, sizeof(U) + (PAIRS ? sizeof(V) : 0) <= 8 
     const U* keys_in, U* keys_out, const V* values_in, V* values_out, const uint32_t* __restrict__ begins,
     const uint32_t* __restrict__ ends, uint32_t num_segments, uint32_t per_group, uint32_t per_wave, uint64_t n, uint32_t bits,
     SegmentBits<U> sort_bits, uint32_t* words) {
-    using Sorter = BlockSort<U, V, PAIRS, kSwBlock, static_cast<int>(kSwMedium / kSwBlock)>;
+    using Sorter = BlockSort<U, V, PAIRS, kSwBlock, static_cast<int>(kSwMedium / kSwBlock), true>;
     constexpr uint32_t kWaveBytes = 1024 + kSwSmall * (sizeof(U) + (PAIRS ? sizeof(V) : 0));
     constexpr uint32_t kLdsBytes = MEDIUM ? sizeof(typename Sorter::Shared) : kSwWaves * kWaveBytes;
     __shared__ __attribute__((aligned(16))) unsigned char s_lds[kLdsBytes];
