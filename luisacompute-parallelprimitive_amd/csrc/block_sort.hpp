@@ -6,7 +6,7 @@
 
 namespace lcpp_hip {
 
-// A pass costs a rank chain of ITEMS dependent LDS round trips per wave, five barriers and one LDS
+// A pass costs a rank chain of ITEMS dependent LDS round trips per wave, four barriers and one LDS
 // exchange, whatever the digits are; digits that are the same in every key of the tile are skipped (a
 // tile of 30-bit codes or of small 64-bit integers takes only the passes that can move anything).
 //
@@ -80,6 +80,7 @@ struct BlockSort {
             if ((static_cast<uint32_t>(vary >> shift) & 0xFFu) == 0) continue;  // the same in every item
 #pragma unroll
             for (uint32_t i = 0; i < kBins / kWave; ++i) cnt[i * kWave + lane] = 0;
+            wave_lds_order();
             uint32_t rank[ITEMS];  // digit << 16 | rank among the wave's items of that digit
             if (!idle) {
 #pragma unroll
@@ -91,6 +92,7 @@ struct BlockSort {
                     const uint32_t base = cnt[d];
                     rank[j] = (d << 16) | (base + below);
                     if ((peers >> lane) == 1ull) cnt[d] = base + below + 1;
+                    wave_lds_order();
                 }
             }
             __syncthreads();

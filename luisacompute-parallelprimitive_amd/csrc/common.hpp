@@ -159,6 +159,12 @@ __device__ __forceinline__ uint32_t popc_lanes_below(uint64_t mask) {
                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
 }
 
+// LDS written by a lane is read by others of its wave: in order in hardware; this keeps the compiler to it.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __ballot(p); }
 
 // Lanes of the wave whose 8-bit digit equals this lane's.  Per digit bit: t = 0 or ~0 (the bit,

@@ -260,6 +260,7 @@ __global__ __launch_bounds__(kBlock, 8) void mid_onesweep_kernel(const K* __rest
     uint32_t* const cnt = s_count[wave];
 #pragma unroll
     for (uint32_t i = 0; i < kDigits / kWave; ++i) cnt[i * kWave + lane] = 0;
+    wave_lds_order();
     uint32_t rank[ITEMS];  // digit << 16 | rank among the wave's keys of that digit
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
@@ -271,6 +272,7 @@ __global__ __launch_bounds__(kBlock, 8) void mid_onesweep_kernel(const K* __rest
         const uint32_t base = cnt[d];
         rank[k] = (d << 16) | (base + below);
         if ((peers >> lane) == 1ull) cnt[d] = base + below + 1;
+        wave_lds_order();
     }
     __syncthreads();
 

@@ -50,12 +50,6 @@ struct WaveLds {
     uint32_t* count;  // 256, 16-byte aligned
 };
 
-// LDS written by a lane is read by others of its wave: in order in hardware; this keeps the compiler to it.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 struct OrOp {
     template <typename T>
     __device__ __forceinline__ T operator()(T a, T b) const { return a | b; }
