@@ -74,7 +74,7 @@ template <typename K, int VB>
 int small_sort(const K* keys_in, K* keys_out, const void* values_in, void* values_out, K* runs_keys, void* runs_values,
                uint32_t n, uint32_t begin_bit, uint32_t end_bit, bool descending, hipStream_t stream);
 
-// mid_sort (radix_mid.hip): onesweep passes with every tile resident, for up to kMidSortMax items.
+// mid_sort (radix_mid.hip): onesweep passes over small tiles that run together, for up to kMidSortMax items.
 constexpr uint32_t kMidSortMax = 1u << 21;
 constexpr int kMidItems = 4;
 constexpr uint32_t kMidTile = 1024 * kMidItems;

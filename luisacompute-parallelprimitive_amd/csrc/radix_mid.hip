@@ -1,4 +1,4 @@
-// Onesweep DeviceRadixSort of medium inputs for gfx950: all tiles of a pass resident at once, one launch for
+// Onesweep DeviceRadixSort of medium inputs for gfx950: the tiles of a pass resident together, one launch for
 // the histogram and one per pass.
 //
 // The large-input passes (radix_sort.hip) are built for throughput: tiles of 14,336 or 18,432 keys leave most
@@ -9,15 +9,19 @@
 //     its end): 40,000 pairs 69.8 -> 33.4 us, 100,003 73.8 -> 38.2, 1,000,003 87.5 -> 60.0, 2,000,003 97.3 ->
 //     79.7; u64 + u32 pairs 109 -> 69, 121 -> 78, 189 -> 122, 220 -> 165.  5, 6 or 8 keys per thread: 61.7, 64.0,
 //     66.7 us at 1,000,003 pairs.  Above 2^21 keys the tiles no longer run together and the large-input passes
-//     are faster (3,000,003 pairs: 116 us here, 105 there).
+//     are faster (3,000,003 pairs: 116 us here, 105 there).  A tile of 8-byte keys with 8-byte values takes 85 KB
+//     of LDS, one workgroup per CU: from 2^20 of them on a pass runs in two rounds, and a call takes about what
+//     the large-input passes take (u64 + u64 pairs there and here: 1,000,003 196.7 and 131.0 us, 1,300,001 207.2
+//     and 198.4, 2,097,152 236.1 and 232.1; all keys equal 224.4 and 230.5).
+//   * Two workgroups per CU leave 64 registers: pairs of 12 bytes spill up to five (1 to 5, by key type and order).
 //   * Histogram workgroups store their digit counts as rows (nothing to clear first); every workgroup of pass
 //     0 adds up the rows of its own pass behind its key loads, and the first ones those of the later passes.
-//   * The digit counts of the tiles before a tile are added up over two levels: groups of 16 tiles,
-//     whose last tile publishes the group's sum in its row (no other tile reads that one's own counts).  A tile reads at most 15 rows of its group and one
-//     row per earlier group, in two steps of which each is one cross-XCD round trip.  (The chained look-back of
-//     the large inputs reads up to one row per earlier tile here, where all tiles publish at the same time:
-//     the reads of the same rows by hundreds of workgroups made a step cost 4 us, 97 us per call of 1,000,003
-//     pairs.)
+//   * The digit counts of the tiles before a tile are added up over two levels: groups of 16 tiles (of 32 up to
+//     32 tiles, where the first level is all there is), whose last tile publishes the group's sum in its row (no
+//     other tile reads that one's own counts).  A tile reads at most 15 (31) rows of its group and one row per
+//     earlier group, in two steps of which each is one cross-XCD round trip.  (The chained look-back of the large
+//     inputs reads up to one row per earlier tile here, where all tiles publish at the same time: the reads of
+//     the same rows by hundreds of workgroups made a step cost 4 us, 97 us per call of 1,000,003 pairs.)
 //   * The rows serve every pass: an entry carries the pass number, so the entries of the pass before read as
 //     unpublished, and the histogram clears them once.
 #include "radix_keys.hpp"
@@ -125,10 +129,14 @@ struct Walk {
     uint32_t* s_count;
     uint32_t* s_row;
 
-    // The sum of this thread's digit over `count` rows, `stride` words apart; row r counts `tiles` tiles from first_tile + r * tiles.
-    // The workgroup polls until all are published; a row still unpublished after `spin_limit` polls is counted
-    // from the keys and published by compare-and-swap, so progress does not depend on the order of dispatch.
-    // (The tiles before another are full.)
+    __device__ __forceinline__ uint32_t digit(U key) const {
+        return static_cast<uint32_t>(sort_bits(twiddle_in<U, KeyTraits<K>::kind, DESC>(key)) >> shift) & 0xFFu;
+    }
+
+    // The sum of this thread's digit over `count` rows, `stride` words apart; row r counts `tiles` tiles from
+    // first_tile + r * tiles.  The workgroup polls until all are published; a row still unpublished after
+    // `spin_limit` polls is counted from the keys and published by compare-and-swap, so progress does not depend on
+    // the order of dispatch.  (The tiles before another are full.)
     __device__ __forceinline__ uint32_t sum(uint32_t* rows, uint32_t stride, uint32_t count, uint32_t first_tile,
                                             uint32_t tiles) const {
         const uint32_t part = threadIdx.x / kDigits;
@@ -157,7 +165,7 @@ struct Walk {
                     const uint32_t r = *s_row - 1u;
                     const U* theirs = reinterpret_cast<const U*>(keys) + (first_tile + r * tiles) * tile_items;
                     for (uint32_t i = threadIdx.x; i < tiles * tile_items; i += kBlock)
-                        atomicAdd(&s_count[static_cast<uint32_t>(sort_bits(twiddle_in<U, KeyTraits<K>::kind, DESC>(theirs[i])) >> shift) & 0xFFu], 1u);
+                        atomicAdd(&s_count[digit(theirs[i])], 1u);
                     __syncthreads();
 #pragma unroll
                     for (int w = 0; w < kWindow; ++w) {
@@ -212,6 +220,8 @@ __global__ __launch_bounds__(kBlock, 8) void mid_onesweep_kernel(const K* __rest
     constexpr int ITEMS = kMidItems;
     constexpr uint32_t TILE = kMidTile;
     static_assert(TILE == static_cast<uint32_t>(kBlock) * ITEMS);
+    constexpr size_t kLds = TILE * (sizeof(U) + VB) + sizeof(uint32_t) * kDigits * (kWaves + 1 + kSplit) + 64;
+    static_assert(sizeof(U) + VB > 12 || 2 * kLds <= (160u << 10), "two workgroups per CU for items of up to 12 bytes");
     __shared__ U s_key[TILE];
     __shared__ VW s_value[VB ? TILE : 1];
     __shared__ uint32_t s_count[kWaves][kDigits];

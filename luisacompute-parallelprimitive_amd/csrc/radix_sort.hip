@@ -1349,7 +1349,7 @@ int sort_entry(void* temp, size_t temp_bytes, const K* keys_in, K* keys_out, con
         if (st == kOk && db) *selector = to;
         return st;
     }
-    // Medium inputs: passes whose tiles are all resident (radix_mid.hip), when the temp storage has room for
+    // Medium inputs: passes over small tiles that run together (radix_mid.hip), when the temp storage has room for
     // their look-back rows (a reference-sized one does).
     if (!hooked && n <= kMidSortMax) {
         MidPlan M;

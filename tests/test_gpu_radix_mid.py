@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 TILE = 4096
 
 
-@pytest.mark.parametrize("dtype,vbytes", [(np.uint32, 0), (np.uint32, 4), (np.float32, 8), (np.uint64, 4), (np.float64, 0)])
+@pytest.mark.parametrize("dtype,vbytes", [(np.uint32, 0), (np.uint32, 4), (np.float32, 8), (np.uint64, 4), (np.float64, 0),
+                                          (np.uint64, 8), (np.int64, 8)])
 @pytest.mark.parametrize("kind", ["uniform", "few"])
 def test_mid_sizes(hip, orc, dev, dtype, vbytes, kind):
     last = LAST[np.dtype(dtype).itemsize]
@@ -83,3 +84,24 @@ def test_mid_smallest_temp_and_in_place(hip, orc, dev, dtype, vbytes):
     hip.sort_pairs(sfx, vbytes, kin, kin, vin, vin, n)
     check_bits(to_host(kin, dtype, n), eko)
     assert np.array_equal(to_host(vin, vals.dtype, n), evo)
+
+
+@pytest.mark.parametrize("spin", [None, 0])
+@pytest.mark.parametrize("dtype", [np.uint64, np.int64])
+def test_mid_more_tiles_than_run_together(hip, orc, dev, dtype, spin):
+    """8-byte keys with 8-byte values, one workgroup per CU: tiles of a second round add up the rows of the first."""
+    n = (1 << 20) + 37 * TILE + 11
+    keys = make_keys(orc, dtype, n, 91, "uniform")
+    vals = np.arange(n, dtype=np.uint64)
+    lib = hip.lib()
+    old = lib.lcpp_hip_get_lookback_spin_limit()
+    try:
+        if spin is not None:
+            lib.lcpp_hip_set_lookback_spin_limit(spin)
+        log(f"mid sort {np.dtype(dtype).name} v8 n={n} spin={spin}")
+        ko, vo = gpu_sort(hip, keys, vals, descending=True)
+    finally:
+        lib.lcpp_hip_set_lookback_spin_limit(old)
+    eko, evo = orc.radix_sort(keys, vals, descending=True)
+    check_bits(ko, eko)
+    assert np.array_equal(vo, evo)
