@@ -39,21 +39,33 @@ def values_for(rng, n, vs):
     return rng.integers(info.min, info.max, n, dtype=dt, endpoint=True)
 
 
-def gpu_scan_by_key(hip, ks, vs, keys, vals, inclusive, init=None, key_mask=-1, in_place=False, op="sum"):
+def full_tiles_temp(hip, n, vs, scan):
+    """Temp storage for the states of full-size tiles (a scan's have no word for the head count) and not for those of the
+    4,096-item tiles that smaller inputs take when there is room."""
+    words = np.dtype(NP[vs]).itemsize // 4
+    nbytes = hip.lib().lcpp_hip_internal_by_key_needed_bytes(n, 4 * words)  # of a reduce: count, sum and claim words
+    state = 8 * (words + 2)
+    if scan:
+        nbytes, state = nbytes // state * (state - 8), state - 8
+    assert nbytes < -(-n // 4096) * state
+    return torch.empty(nbytes // 4, dtype=torch.int32, device="cuda:0")
+
+
+def gpu_scan_by_key(hip, ks, vs, keys, vals, inclusive, init=None, key_mask=-1, in_place=False, op="sum", temp=None):
     n = keys.size
     d_k, d_v = to_dev(keys), to_dev(vals)
     d_o = d_v if in_place else torch.empty_like(d_v)
-    hip.scan_by_key(ks, vs, d_k, d_v, d_o, n, inclusive=inclusive, init=init, key_mask=key_mask, op=op)
+    hip.scan_by_key(ks, vs, d_k, d_v, d_o, n, inclusive=inclusive, init=init, key_mask=key_mask, op=op, temp=temp)
     return to_host(d_o, NP[vs], n)
 
 
-def gpu_reduce_by_key(hip, ks, vs, keys, vals, key_mask=-1, op="sum"):
+def gpu_reduce_by_key(hip, ks, vs, keys, vals, key_mask=-1, op="sum", temp=None):
     n = keys.size
     d_k, d_v = to_dev(keys), to_dev(vals)
     uniq = fill_dev(max(n, 1), keys.itemsize, 0x5A5A5A5A)
     agg = fill_dev(max(n, 1), vals.itemsize, 0x5A5A5A5A)
     runs = fill_dev(1, 4, 17)
-    hip.reduce_by_key(ks, vs, d_k, d_v, uniq, agg, runs, n, key_mask=key_mask, op=op)
+    hip.reduce_by_key(ks, vs, d_k, d_v, uniq, agg, runs, n, key_mask=key_mask, op=op, temp=temp)
     r = int(to_host(runs, np.uint32, 1)[0])
     return to_host(uniq, keys.dtype, r), to_host(agg, NP[vs], r), r
 
@@ -225,11 +237,13 @@ def test_in_place_scan_with_forced_fallback(hip, orc, dev, vs):
     try:
         lib.lcpp_hip_set_lookback_spin_limit(0)
         for inclusive in (True, False):
-            log(f"in-place fallback {vs} inclusive={inclusive}")
-            got = gpu_scan_by_key(hip, "i32", vs, keys, vals, inclusive, None if inclusive else 0, in_place=True)
-            check_scan(orc, keys, vals, got, vs, inclusive, None if inclusive else 0, -1)
-        uniq, agg, runs = gpu_reduce_by_key(hip, "i32", vs, keys, vals)
-        check_reduce(orc, keys, vals, uniq, agg, runs, vs, -1)
+            for temp in (None, full_tiles_temp(hip, n, vs, scan=True)):
+                log(f"in-place fallback {vs} inclusive={inclusive} full-size tiles={temp is not None}")
+                got = gpu_scan_by_key(hip, "i32", vs, keys, vals, inclusive, None if inclusive else 0, in_place=True, temp=temp)
+                check_scan(orc, keys, vals, got, vs, inclusive, None if inclusive else 0, -1)
+        for temp in (None, full_tiles_temp(hip, n, vs, scan=False)):
+            uniq, agg, runs = gpu_reduce_by_key(hip, "i32", vs, keys, vals, temp=temp)
+            check_reduce(orc, keys, vals, uniq, agg, runs, vs, -1)
     finally:
         lib.lcpp_hip_set_lookback_spin_limit(old)
 
@@ -396,11 +410,15 @@ def test_minmax_by_key_long_runs_and_fallback(hip, orc, dev, op):
         for spin in (old, 0):
             lib.lcpp_hip_set_lookback_spin_limit(spin)
             log(f"by_key {op} long runs spin={spin}")
-            got = gpu_scan_by_key(hip, "i32", "f32", keys, vals, True, op=op)
-            assert same_bits(got, orc.scan_by_key_minmax(op, keys, vals, True))
-            uniq, agg, runs = gpu_reduce_by_key(hip, "i32", "f32", keys, vals, op=op)
+            want = orc.scan_by_key_minmax(op, keys, vals, True)
             ou, oa = orc.reduce_by_key_minmax(op, keys, vals)
-            assert runs == ou.size and same_bits(agg, oa)
+            for full in (False, True):
+                temp = full_tiles_temp(hip, n, "f32", scan=True) if full else None
+                got = gpu_scan_by_key(hip, "i32", "f32", keys, vals, True, op=op, temp=temp)
+                assert same_bits(got, want)
+                temp = full_tiles_temp(hip, n, "f32", scan=False) if full else None
+                uniq, agg, runs = gpu_reduce_by_key(hip, "i32", "f32", keys, vals, op=op, temp=temp)
+                assert runs == ou.size and same_bits(agg, oa)
     finally:
         lib.lcpp_hip_set_lookback_spin_limit(old)
 

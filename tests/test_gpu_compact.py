@@ -528,7 +528,9 @@ def test_errors(hip, dev):
 
 
 # ---- the register-resident rows kernel (selects and partitions not in place) and the staging kernel ----
-R4, R8, R4F, R8F = 16384, 6144, 12288, 6144  # rows-kernel tiles: 4- / 8-byte items, without / with flags
+# Rows-kernel tiles of inputs of these sizes: 4- / 8-byte items, without / with flags.  Larger inputs' tiles:
+# test_gpu_tile_sizes.py.
+R4, R8, R4F, R8F = 4096, 2048, 4096, 2048
 
 
 @pytest.fixture(params=[True, False], ids=["rows", "staging"])

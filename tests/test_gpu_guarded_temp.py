@@ -111,7 +111,7 @@ def _sorted_check(got, keys):
     assert same_bits(got[keys.size:], np.full(SENTINEL_ITEMS, sentinel(keys.dtype), keys.dtype))
 
 
-@pytest.mark.parametrize("n", [5000, (1 << 22) + 5])
+@pytest.mark.parametrize("n", [5000, 300_007, (1 << 22) + 5])
 def test_reduce_scan_sort_spmv_stay_inside_their_temp(hip, orc, dev, n):
     rng = np.random.default_rng(n)
     log(f"guarded temp: reduce / scan / sort / spmv n={n}")
@@ -182,7 +182,7 @@ def test_reduce_scan_sort_spmv_stay_inside_their_temp(hip, orc, dev, n):
     assert same_bits(to_host(y, np.float32)[rows:], np.full(SENTINEL_ITEMS, sentinel(np.float32), np.float32))
 
 
-@pytest.mark.parametrize("n", [5000, (1 << 22) + 5])
+@pytest.mark.parametrize("n", [5000, 300_007, (1 << 22) + 5])
 def test_by_key_compaction_segmented_stay_inside_their_temp(hip, orc, dev, n):
     rng = np.random.default_rng(n + 1)
     log(f"guarded temp: by-key / compaction / segmented n={n}")

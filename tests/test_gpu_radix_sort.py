@@ -275,20 +275,21 @@ def test_benchmark_sort_pairs_2p27(hip, orc, dev, kind):
     complete_stable_check(to_host(k, np.uint64), to_host(ko, np.uint64), to_host(vo, np.uint32))
 
 
-@pytest.mark.parametrize("kdtype,vbytes,descending,n", [(np.uint32, 0, False, (1 << 20) + 4321),
-                                                        (np.uint32, 4, True, (1 << 20) + 4321),
-                                                        (np.uint64, 4, False, (1 << 20) + 4321),
-                                                        (np.float32, 0, True, (1 << 20) + 4321),
+@pytest.mark.parametrize("kdtype,vbytes,descending,n", [(np.uint32, 0, False, (1 << 21) + 4321),
+                                                        (np.uint32, 4, True, (1 << 21) + 4321),
+                                                        (np.uint64, 4, False, (1 << 21) + 4321),
+                                                        (np.uint64, 8, True, (1 << 21) + 4321),
+                                                        (np.float32, 0, True, (1 << 21) + 4321),
                                                         (np.uint32, 0, False, (1 << 23) + 17)])
 def test_forced_lookback_fallback(hip, orc, dev, kdtype, vbytes, descending, n):
-    """Spin limit 0: every unpublished predecessor's digit counts are computed by the waiting
+    """Spin limit 0, sizes above the medium sorts': every unpublished predecessor's digit counts are computed by the waiting
     workgroup from that tile's keys and published by compare-and-swap (the largest case walks back
     over hundreds of tiles, several look-back steps per tile)."""
     lib = hip.lib()
     log(f"sort forced fallback {kdtype.__name__} vbytes={vbytes} desc={descending}")
     raw = orc.generate(0, n, 808)
     keys = raw.copy() if kdtype == np.uint64 else (raw >> np.uint64(32)).astype(np.uint32).view(kdtype).copy()
-    vals = None if vbytes == 0 else np.arange(n, dtype=np.uint32)
+    vals = None if vbytes == 0 else np.arange(n, dtype=np.uint32 if vbytes == 4 else np.uint64)
     old = lib.lcpp_hip_get_lookback_spin_limit()
     try:
         lib.lcpp_hip_set_lookback_spin_limit(0)
@@ -310,7 +311,7 @@ def test_rank_modes_agree_with_oracle(hip, orc, dev, mode, case):
     split between them) gives the stable ranks; low-entropy keys put many lanes of a wave on the same
     digit entry."""
     lib = hip.lib()
-    n = 500009
+    n = (1 << 21) + 9  # above the medium sorts', which the default mode would take
     raw = orc.generate(0, n, 4040)
     vals = np.arange(n, dtype=np.uint32)
     desc = case.endswith("desc")
@@ -342,29 +343,29 @@ def test_first_pass_offsets_from_histogram(hip, orc, dev, precount, case):
     """The first pass takes its tile offsets from the histogram's per-tile counts (precount 1, for a single
     portion with aligned keys) or walks the look-back like the other passes (0, the default): the same
     stable order either way, for full and partial bit ranges, a partial last tile, pairs, descending
-    order and the DoubleBuffer form."""
+    order and the DoubleBuffer form (sizes above the medium sorts')."""
     lib = hip.lib()
-    raw = orc.generate(0, 1 << 20, 5150)
+    raw = orc.generate(0, (1 << 21) + (1 << 16), 5150)
     try:
         old = lib.lcpp_hip_internal_radix_precount(precount)
         if case == "u32_random":
             keys = (raw >> np.uint64(32)).astype(np.uint32)
             check_bits(gpu_sort(hip, keys), orc.radix_sort(keys))
         elif case == "u64_pairs_desc":
-            keys = raw[:300007] & np.uint64(0x0F0F0F0F0F0F0F0F)
+            keys = raw[:(1 << 21) + 7] & np.uint64(0x0F0F0F0F0F0F0F0F)
             vals = np.arange(keys.size, dtype=np.uint32)
             ko, vo = gpu_sort(hip, keys, vals, descending=True)
             eko, evo = orc.radix_sort(keys, vals, descending=True)
             check_bits(ko, eko)
             assert np.array_equal(vo, evo)
         elif case == "f32_bits_3_29":
-            keys = orc.generate(6, 250001, 5151)
+            keys = orc.generate(6, (1 << 21) + 50_001, 5151)
             check_bits(gpu_sort(hip, keys, begin_bit=3, end_bit=29), orc.radix_sort(keys, begin_bit=3, end_bit=29))
         elif case == "i32_partial_tile":
-            keys = (raw[:16384 * 7 + 1234] >> np.uint64(40)).astype(np.int32) - (1 << 23)
+            keys = (raw[:16384 * 130 + 1234] >> np.uint64(40)).astype(np.int32) - (1 << 23)
             check_bits(gpu_sort(hip, keys), orc.radix_sort(keys))
         else:
-            n = 1 << 19
+            n = (1 << 21) + (1 << 15)
             keys = (raw[:n] >> np.uint64(16)).astype(np.uint32)
             d0, d1 = to_dev(keys), fill_dev(n, 4, -1)
             sel = hip.sort_keys_db("u32", d0, d1, 0, n)

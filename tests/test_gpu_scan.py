@@ -20,12 +20,19 @@ REGRESSION_SIZES = [1, 31, 32, 33, 255, 256, 257, 3839, 3840, 3841, 4095, 4096, 
                     262147]
 
 
-def gpu_scan(hip, suffix, a, inclusive=False, init=None, offset_in=0, offset_out=0):
+def single_pass_temp(hip, n, itemsize):
+    """The smallest temp storage a scan accepts: no room for the small scans' tile totals, so it takes the single pass."""
+    nbytes = hip.lib().lcpp_hip_internal_scan_needed_bytes(n, itemsize)
+    assert n > 65536 // itemsize and nbytes < -(-n // (16384 // itemsize)) * itemsize
+    return torch.empty(nbytes // 4, dtype=torch.int32, device="cuda:0")
+
+
+def gpu_scan(hip, suffix, a, inclusive=False, init=None, offset_in=0, offset_out=0, temp=None):
     n = a.size - offset_in
     d_in = to_dev(a)[offset_in:]
     out_full = fill_dev(n + offset_out, a.dtype.itemsize, 0x7E7E7E7E)
     d_out = out_full[offset_out:]
-    hip.scan_sum(suffix, d_in, d_out, n, inclusive=inclusive, init=init)
+    hip.scan_sum(suffix, d_in, d_out, n, inclusive=inclusive, init=init, temp=temp)
     return to_host(out_full, a.dtype)[offset_out:offset_out + n]
 
 
@@ -121,13 +128,14 @@ def forced_fallback(hip):
         lib.lcpp_hip_set_lookback_spin_limit(old)
 
 
-@pytest.mark.parametrize("n", [4097, 65536 * 3 + 5, (1 << 22) + 77])
+@pytest.mark.parametrize("n", [24577, 65536 * 3 + 5, (1 << 22) + 77])
 def test_forced_fallback_integer(hip, orc, dev, forced_fallback, n):
     log(f"scan forced fallback n={n}")
     a = orc.generate(1, n, n)
+    temp = single_pass_temp(hip, n, 4)
     for inclusive in (False, True):
-        assert np.array_equal(gpu_scan(hip, "u32", a, inclusive), orc.scan_sum_u32(a, inclusive))
-    assert np.array_equal(gpu_scan(hip, "u32", a, False, offset_in=1), orc.scan_sum_u32(a[1:]))
+        assert np.array_equal(gpu_scan(hip, "u32", a, inclusive, temp=temp), orc.scan_sum_u32(a, inclusive))
+    assert np.array_equal(gpu_scan(hip, "u32", a, False, offset_in=1, temp=temp), orc.scan_sum_u32(a[1:]))
 
 
 def test_forced_fallback_float_within_tolerance(hip, orc, dev, forced_fallback):
@@ -135,17 +143,17 @@ def test_forced_fallback_float_within_tolerance(hip, orc, dev, forced_fallback):
     # decoupled look-back), so the check is the order-independent bound of test_float_within_tolerance.
     n = (1 << 22) + 123
     a = orc.generate(6, n, 5)
-    got = gpu_scan(hip, "f32", a).astype(np.float64)
+    got = gpu_scan(hip, "f32", a, temp=single_pass_temp(hip, n, 4)).astype(np.float64)
     exact, absum = orc.scan_sum_f32(a)
     bound = (np.arange(n) + 2) * np.finfo(np.float32).eps * absum
     assert np.all(np.abs(got - exact) <= bound)
 
 
-def gpu_scan_in_place(hip, suffix, a, inclusive=False, init=None):
+def gpu_scan_in_place(hip, suffix, a, inclusive=False, init=None, temp=None):
     """Scans `a` with d_in == d_out, as the reference's InclusiveScanInit test does
     (tests/device_scan_test.cpp:288-321)."""
     d = to_dev(a)
-    hip.scan_sum(suffix, d, d, a.size, inclusive=inclusive, init=init)
+    hip.scan_sum(suffix, d, d, a.size, inclusive=inclusive, init=init, temp=temp)
     return to_host(d, a.dtype)
 
 
@@ -168,7 +176,8 @@ def test_in_place_forced_fallback(hip, orc, dev, forced_fallback, n):
     log(f"scan in-place forced fallback n={n}")
     a = orc.generate(1, n, n + 2)
     for inclusive in (False, True):
-        assert np.array_equal(gpu_scan_in_place(hip, "u32", a, inclusive), orc.scan_sum_u32(a, inclusive))
+        got = gpu_scan_in_place(hip, "u32", a, inclusive, temp=single_pass_temp(hip, n, 4))
+        assert np.array_equal(got, orc.scan_sum_u32(a, inclusive))
 
 
 # ---- 8-byte items --------------------------------------------------------------------------------
@@ -236,10 +245,11 @@ def test_64bit_forced_fallback(hip, orc, dev, forced_fallback, n):
     """Claimed predecessors publish both words of their state; readers accept only matching pairs."""
     log(f"scan u64 forced fallback n={n}")
     a = orc.generate(0, n, n + 9)
+    temp = single_pass_temp(hip, n, 8)
     for inclusive in (False, True):
-        assert np.array_equal(gpu_scan(hip, "u64", a, inclusive), orc.scan_sum_u64(a, inclusive))
+        assert np.array_equal(gpu_scan(hip, "u64", a, inclusive, temp=temp), orc.scan_sum_u64(a, inclusive))
     b = np.ones(n, np.float64)
-    assert gpu_scan(hip, "f64", b, inclusive=True).tolist() == [float(i + 1) for i in range(n)]
+    assert gpu_scan(hip, "f64", b, inclusive=True, temp=temp).tolist() == [float(i + 1) for i in range(n)]
 
 
 @pytest.mark.parametrize("n", [TILE64 * 5 + 3, (1 << 22) + 77])
@@ -247,7 +257,8 @@ def test_64bit_in_place_forced_fallback(hip, orc, dev, forced_fallback, n):
     log(f"scan u64 in-place forced fallback n={n}")
     a = orc.generate(0, n, n + 13)
     for inclusive in (False, True):
-        assert np.array_equal(gpu_scan_in_place(hip, "u64", a, inclusive), orc.scan_sum_u64(a, inclusive))
+        got = gpu_scan_in_place(hip, "u64", a, inclusive, temp=single_pass_temp(hip, n, 8))
+        assert np.array_equal(got, orc.scan_sum_u64(a, inclusive))
 
 
 # ---- min / max operators -------------------------------------------------------------------------
@@ -258,11 +269,11 @@ MINMAX_SUFFIX = {"i32": np.int32, "u32": np.uint32, "f32": np.float32, "i64": np
 TILE32 = 24576  # 4-byte items per scan tile
 
 
-def gpu_scan_minmax(hip, op, suffix, a, inclusive=False, init=None):
+def gpu_scan_minmax(hip, op, suffix, a, inclusive=False, init=None, temp=None):
     n = a.size
     d_in = to_dev(a)
     d_out = fill_dev(n, a.dtype.itemsize, 0x7E7E7E7E)
-    hip.scan_minmax(op, suffix, d_in, d_out, n, inclusive=inclusive, init=init)
+    hip.scan_minmax(op, suffix, d_in, d_out, n, inclusive=inclusive, init=init, temp=temp)
     return to_host(d_out, a.dtype)
 
 
@@ -311,8 +322,9 @@ def test_scan_minmax_monotone(hip, orc, dev, suffix):
     a = np.arange(n, 0, -1).astype(MINMAX_SUFFIX[suffix])
     for op in ("min", "max"):
         for inclusive in (False, True):
-            got = gpu_scan_minmax(hip, op, suffix, a, inclusive)
-            assert same_bits(got, orc.scan_minmax(op, a, inclusive))
+            want = orc.scan_minmax(op, a, inclusive)
+            for temp in (None, single_pass_temp(hip, n, a.itemsize)):
+                assert same_bits(gpu_scan_minmax(hip, op, suffix, a, inclusive, temp=temp), want)
 
 
 @pytest.mark.parametrize("suffix", ["f32", "f64"])
@@ -329,9 +341,11 @@ def test_scan_minmax_signed_zero_order(hip, orc, dev, suffix):
     b[0] = -0.0
     for op in ("min", "max"):
         for x in (a, b):
-            got = gpu_scan_minmax(hip, op, suffix, x, inclusive=True)
-            assert same_bits(got, orc.scan_minmax(op, x, inclusive=True))
-            assert np.all(np.signbit(got) == np.signbit(x[0]))
+            want = orc.scan_minmax(op, x, inclusive=True)
+            for temp in (None, single_pass_temp(hip, n, a.itemsize)):
+                got = gpu_scan_minmax(hip, op, suffix, x, inclusive=True, temp=temp)
+                assert same_bits(got, want)
+                assert np.all(np.signbit(got) == np.signbit(x[0]))
 
 
 @pytest.mark.parametrize("suffix", ["u32", "f32", "i64", "f64"])
@@ -340,14 +354,15 @@ def test_scan_minmax_forced_fallback(hip, orc, dev, forced_fallback, suffix):
     n = (1 << 22) + 77
     log(f"scan minmax forced fallback {suffix}")
     a = minmax_input(suffix, n, 23)
+    temp = single_pass_temp(hip, n, a.itemsize)
     for op in ("min", "max"):
         for inclusive in (False, True):
-            got = gpu_scan_minmax(hip, op, suffix, a, inclusive)
+            got = gpu_scan_minmax(hip, op, suffix, a, inclusive, temp=temp)
             assert same_bits(got, orc.scan_minmax(op, a, inclusive))
     if suffix.startswith("f"):
         z = np.full(n, -0.0, MINMAX_SUFFIX[suffix])
         z[0] = 0.0
-        assert not np.any(np.signbit(gpu_scan_minmax(hip, "min", suffix, z, inclusive=True)))
+        assert not np.any(np.signbit(gpu_scan_minmax(hip, "min", suffix, z, inclusive=True, temp=temp)))
 
 
 def test_scan_minmax_all_nan_prefix(hip, orc, dev):
@@ -379,7 +394,7 @@ def test_scan_minmax_in_place_forced_fallback(hip, orc, dev, forced_fallback):
     for suffix in ("i32", "f64"):
         a = minmax_input(suffix, n, 31)
         d = to_dev(a)
-        hip.scan_minmax("min", suffix, d, d, n, inclusive=True)
+        hip.scan_minmax("min", suffix, d, d, n, inclusive=True, temp=single_pass_temp(hip, n, a.itemsize))
         assert same_bits(to_host(d, a.dtype), orc.scan_minmax("min", a, inclusive=True))
 
 
