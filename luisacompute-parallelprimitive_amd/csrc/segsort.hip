@@ -11,12 +11,14 @@
 // leaves a DoubleBuffer untouched.  Any stable sort by the same order gives the same output, so the
 // sort here is free to differ from the reference's merge passes.
 //
-// MI355X design (radix orders with many short segments, and value orders; see wave_route for the others):
+// MI355X design (radix orders with many short segments, and value orders; see wave_route for the others, whose
+// medium segments may take the block kernel too: medium_apart):
 //   * Block phase: chunks sorted in LDS by one 256-thread workgroup each, C = 4,096 items in radix
 //     order and 2,048 in value order.  Tiny segments (<= 16 items) are sorted by one thread each, in
 //     registers; small ones (<= 512 items) together per 2,048-item tile of the item range (a joint sort
-//     with position labels when a tile holds more than two), medium ones (<= C) by one workgroup each, and long ones chunk by chunk by a grid-stride
-//     kernel over C-item tiles, so neither many tiny segments nor a few long ones leave the GPU idle.
+//     with position labels when a tile holds more than two), medium ones (<= C) by one workgroup each, and
+//     long ones chunk by chunk by a grid-stride kernel over C-item tiles, so neither many tiny segments nor
+//     a few long ones leave the GPU idle.
 //   * Radix order, medium segments and chunks: a stable LSD radix sort in LDS, 8-bit digits, 4, 8 or
 //     16 items per thread by length; per pass a ballot match ranks each wave's items against per-wave
 //     digit counters, one workgroup scan orders (digit, wave), items are scattered to LDS and read back.

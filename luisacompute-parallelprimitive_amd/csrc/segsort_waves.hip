@@ -10,7 +10,7 @@
 //     lane follow the length (1, 2, 4 or 8), since a rank step costs the same whether its items are real.
 //   * Tiny segments (up to 16 items) take a 16-lane row each, four at a time.
 //   * Medium segments are collected by the workgroup's waves and sorted by all 512 threads, 2, 4 or 8 items per
-//     thread.
+//     thread (of narrow items in large inputs by segsort.hip's block kernel: medium_apart).
 //   * Digits that are the same in a whole segment are skipped.
 // The kinds of key differ by two mask words, so the code exists once per key and value size.
 #include "block_sort.hpp"
