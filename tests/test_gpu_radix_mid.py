@@ -87,7 +87,7 @@ def test_mid_smallest_temp_and_in_place(hip, orc, dev, dtype, vbytes):
 
 
 @pytest.mark.parametrize("spin", [None, 0])
-@pytest.mark.parametrize("dtype", [np.uint64, np.int64])
+@pytest.mark.parametrize("dtype", [np.uint64, np.int64, np.float64])
 def test_mid_more_tiles_than_run_together(hip, orc, dev, dtype, spin):
     """8-byte keys with 8-byte values, one workgroup per CU: tiles of a second round add up the rows of the first."""
     n = (1 << 20) + 37 * TILE + 11
