@@ -112,10 +112,13 @@ def test_double_buffer_in_place(hip, orc, dev, step, longest):
     np.testing.assert_array_equal(to_host(v0, np.uint32, n), wv)
 
 
-def test_segments_on_both_sides_of_2p31(hip, dev):
-    """Offsets that a signed 32-bit word does not hold: one segment for each number of items per lane, and medium ones."""
+@pytest.mark.parametrize("vb", [4, 8])
+def test_segments_on_both_sides_of_2p31(hip, dev, vb):
+    """Offsets that a signed 32-bit word does not hold: one segment for each number of items per lane, tiny and medium ones
+    (which 12-byte items keep in the wave kernel)."""
     n = (1 << 31) + 20_000
-    lengths = [40, 100, 200, 300, 512, 900, 4096]
+    lengths = [1, 9, 40, 100, 200, 300, 512, 900, 4096]
+    v_t = torch.int32 if vb == 4 else torch.int64
     b, e, at = [], [], (1 << 31) - sum(lengths) - 100
     for x in lengths + [333] + lengths:  # the one in the middle straddles 2^31
         b.append(at)
@@ -127,12 +130,12 @@ def test_segments_on_both_sides_of_2p31(hip, dev):
     some = rng.integers(0, 1 << 32, last - first, dtype=np.uint64).astype(np.uint32)
     keys = torch.zeros(n, dtype=torch.int32, device=dev)
     keys[first:last] = to_dev(some)
-    vals = torch.zeros(n, dtype=torch.int32, device=dev)
-    vals[first:last] = torch.arange(last - first, dtype=torch.int32, device=dev)
+    vals = torch.zeros(n, dtype=v_t, device=dev)
+    vals[first:last] = torch.arange(last - first, dtype=v_t, device=dev)
     ko, vo = torch.full_like(keys, -1), torch.full_like(vals, -1)
     hip.segmented_sort("u32", keys, ko, n, len(b), to_dev(np.array(b, np.uint32)), to_dev(np.array(e, np.uint32)),
                        values_in=vals, values_out=vo)
-    wk, wv = np.full(last - first, 0xFFFFFFFF, np.uint32), np.full(last - first, -1, np.int32)
+    wk, wv = np.full(last - first, 0xFFFFFFFF, np.uint32), np.full(last - first, -1, np.int64)
     for x, y in zip(b, e):
         order = np.argsort(some[x - first:y - first], kind="stable")
         wk[x - first:y - first] = some[x - first:y - first][order]
